@@ -259,7 +259,7 @@ constexpr TileCfg kTiles[] = {{2, 3}, {2, 2}, {2, 1}, {1, 2}, {1, 1}};
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
 // Variant code: bit 14 = split f32 products, bits 13..9 = GemmLayouts::io
-// (bf16-stored operands and split copies, the instances of k_gemm_io*.hip),
+// (bf16-stored operands, the instances of k_gemm_io*.hip),
 // bit 8 = bf16 MFMA (autocast), bit 7 =
 // grouped accumulation, bit 6 = GELU epilogues, bit 5 = mapped operands,
 // bit 4 = LDS-DMA path, bits 3..0 = transA, transB, vecA, vecB.
@@ -362,6 +362,17 @@ int g_split_target = 0;    // workgroups a split-K launch aims for; 0: model
 bool g_allow_dma = true;   // LDS-DMA path where the shape allows it
 int g_f32_x3 = -1;         // f32 GEMMs as split bf16 products; -1: read MALUS_F32_GEMM once
 
+void read_forced_tile() {
+  if (g_forced_tile != -2) return;
+  g_forced_tile = -1;  // MALUS_GEMM_TILE=TMxTN pins a tile (tuning sweeps)
+  if (const char* e = getenv("MALUS_GEMM_TILE"))
+    for (int i = 0; i < kNumTiles; ++i) {
+      char buf[8];
+      snprintf(buf, sizeof(buf), "%dx%d", kTiles[i].tm, kTiles[i].tn);
+      if (!strcmp(buf, e)) g_forced_tile = i;
+    }
+}
+
 // Default on; MALUS_F32_GEMM=fp32 starts the process on the FP32 MFMA.
 bool f32_x3() {
   if (g_f32_x3 < 0) {
@@ -378,20 +389,9 @@ bool f32_x3() {
 // GEMMs, K = tokens) split K so the grid fills the chip's workgroup slots.
 // tri: A lower-triangular (GemmLayouts::tri_a); a tile row then runs on
 // average (n + 1) / (2 n) of K for n tile rows, which favours short tiles.
-// bf: the launch runs on the bf16 MFMA (autocast, or bf16-stored operands);
-// x3: the f32 product as split bf16 pieces (LDS-DMA kernels); groups: the
-// products one grouped launch runs side by side.
-Plan plan_gemm(int batch, int M, int N, int K, int v, bool tri = false, int only_tile = -1, bool bf = false,
-               bool x3 = false, int groups = 1) {
-  if (g_forced_tile == -2) {  // MALUS_GEMM_TILE=TMxTN pins a tile (tuning sweeps)
-    g_forced_tile = -1;
-    if (const char* e = getenv("MALUS_GEMM_TILE"))
-      for (int i = 0; i < kNumTiles; ++i) {
-        char buf[8];
-        snprintf(buf, sizeof(buf), "%dx%d", kTiles[i].tm, kTiles[i].tn);
-        if (!strcmp(buf, e)) g_forced_tile = i;
-      }
-  }
+// bf: the launch runs on the bf16 MFMA (autocast, or bf16-stored operands).
+Plan plan_gemm(int batch, int M, int N, int K, int v, bool tri = false, int only_tile = -1, bool bf = false) {
+  read_forced_tile();
   constexpr double kCuRate = 157.3e12 / 256 * 0.75;  // FLOP/s per CU
   constexpr double kHbm = 4.0e12;                     // B/s for the partials
   Plan best{0, 1, K};
@@ -403,22 +403,8 @@ Plan plan_gemm(int batch, int M, int N, int K, int v, bool tri = false, int only
   // time, and the 128x192 tile (more MFMA work per staged byte) with the
   // cost model's split measured 10-20 % faster on the same shapes.
   const bool wgrad = (v & 16) && (v & 8) && batch == 1 && K >= 4096 && g_forced_tile < 0 && g_split_target == 0;
-  // The split f32 product (six bf16 MFMAs per staged f32 slab) favours
-  // wider tiles (fewer staged bytes per product) where the grid still fills
-  // the chip.  Per call in the C5 step (kernel trace, 128x64 against the
-  // wider tile): the three grouped q/k/v weight gradients 124 -> 114 us on
-  // 128x128 with the cost model's split.  The single 384x384 weight
-  // gradient (41 against 53 us), the 1536-wide ones, the GELU VJP (160
-  // against 226 us: the wider tiles lose its epilogue prefetch) and the
-  // K = 1536, N = 384 products keep the f32 plan (128x128 with a split of 2
-  // gained 3-7 us a call before the forward GEMMs read split weights, and
-  // measured 0.3 % slower on the step after); the GELU forward takes
-  // 128x192 (153 -> 135 us) from the caller.
-  const bool wgrad_bf = wgrad && (g_autocast || bf || (x3 && groups > 1));
-  if (wgrad_bf) only_tile = x3 && !g_autocast && !bf ? 1 : 0;  // kTiles[0] = 128x192, kTiles[1] = 128x128
-  // the occupancy the cost model sees: the split kernels' own for the wide
-  // tiles picked above (it sets their K split), else the f32 kernels'
-  const int occ_v = x3 && only_tile >= 0 ? (v & ~64) | kVarX3 : v & ~64;
+  const bool wgrad_bf = wgrad && (g_autocast || bf);
+  if (wgrad_bf) only_tile = 0;
   for (int ti = 0; ti < kNumTiles; ++ti) {
     if (g_forced_tile >= 0 && ti != g_forced_tile) continue;
     if (only_tile >= 0 && g_forced_tile < 0 && ti != only_tile) continue;
@@ -427,7 +413,7 @@ Plan plan_gemm(int batch, int M, int N, int K, int v, bool tri = false, int only
         !((kTiles[ti].tm == 2 && kTiles[ti].tn == 1) || (kTiles[ti].tm == 1 && kTiles[ti].tn == 2)))
       continue;
     const long tiles = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch;
-    const int occ = occupancy(ti, occ_v);
+    const int occ = occupancy(ti, v & ~64);
     int cand[3] = {1, 1, 1};
     if (batch == 1 && K >= 1024) {
       const int max_split = K / 512;  // >= 32 K steps per workgroup amortize its prologue and partial tile
@@ -455,17 +441,75 @@ Plan plan_gemm(int batch, int M, int N, int K, int v, bool tri = false, int only
   return best;
 }
 
+// ---- split products, split once per workgroup (k_gemm_x3.h) ------------------
+// The tiles with their threads, the workgroups of a CU, and the time in us
+// of one 16-deep slab: of the first workgroup of a CU (lat) and of each
+// further one there (thr).  Measured on 16384 x 384 x 1536 and its transposes
+// (128x192: 103-110 us for one workgroup of 96 slabs per CU), 8192 x 1024 x
+// 4096 (128x128: 350 us, 256x128: 320 us) and 256 x 384 x 384 (64x64: 12 us
+// for 24 slabs, one workgroup on some CUs).  The wide tiles split fewer values and
+// read fewer fragments per product; which of them wins is the busiest CU's
+// share of the tiles.
+struct X3Tile { int bm, bn, threads, conc; double lat, thr; };
+constexpr X3Tile kX3Tiles[] = {{128, 192, 256, 2, 1.0, 1.0},
+                               {128, 128, 256, 2, 0.66, 0.66},
+                               {256, 128, 512, 1, 1.25, 1.25},
+                               {64, 64, 256, 4, 0.33, 0.24}};
+
+// The tile and K split with the smallest modelled time of the busiest CU,
+// plus the split-K partials' round trip.  ti < 0: the kernels of
+// k_gemm_dma.h, which keep the batched products (the composed attention's,
+// K = T or the head size), K < 128 (the two slabs in flight are then most of
+// the K loop: 2048 x 512 x 128 takes 7.4 us here and 7.2 there) and the tuning
+// knobs' tiles and splits.
+// groups: the products one grouped launch runs side by side.  They do not
+// change a split, so that a grouped product has the bits of the single one.
+Plan plan_x3(int batch, int M, int N, int K, bool split_ok, int groups) {
+  Plan best{-1, 1, K};
+  read_forced_tile();
+  if (g_forced_tile >= 0 || g_split_target > 0 || batch > 1 || K < 128) return best;
+  if (split_ok) groups = 1;
+  double best_t = 1e300;
+  for (int ti = 0; ti < (int)(sizeof(kX3Tiles) / sizeof(kX3Tiles[0])); ++ti) {
+    const X3Tile& c = kX3Tiles[ti];
+    const long tiles = (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * groups;
+    for (int per = 0; per <= 3; ++per) {  // no split, or about `per` workgroups per CU
+      long sp = 1;
+      if (per > 0) {
+        sp = per * 256 / tiles;
+        if (sp > K / 256) sp = K / 256;
+        if (!split_ok || K < 1024 || sp < 2) continue;
+      }
+      const int kc = (int)((K + sp - 1) / sp + BK - 1) / BK * BK;
+      const int ns = (K + kc - 1) / kc;
+      const long per_cu = (tiles * ns + 255) / 256;
+      const long rounds = (per_cu + c.conc - 1) / c.conc;
+      // 3 us a round for the first loads and the stores of C
+      double t = 1e-6 * (kc / BK) * (rounds * c.lat + (per_cu - rounds) * c.thr) + rounds * 3e-6;
+      if (ns > 1) t += (ns + 1.0) * M * N * groups * 4.0 / 4e12 + 3e-6;
+      if (t < best_t * 0.999) { best_t = t; best = Plan{ti, ns, kc}; }
+    }
+  }
+  return best;
+}
+
+// The launch of a plan: the tile's size and threads on either path.
+struct TileShape { int bm, bn; unsigned threads; };
+TileShape tile_shape(bool once, int ti) {
+  if (once) return TileShape{kX3Tiles[ti].bm, kX3Tiles[ti].bn, (unsigned)kX3Tiles[ti].threads};
+  return TileShape{64 * kTiles[ti].tm, 64 * kTiles[ti].tn, 256};
+}
+
 }  // namespace
 
 namespace {
 
-void trace_plan(int batch, int M, int N, int K, bool transA, bool transB, bool dma, const Plan& p, int v,
-                const char* tag) {
+void trace_plan(int batch, int M, int N, int K, bool transA, bool transB, const char* path, const Plan& p,
+                const TileShape& t, const char* tag) {
   static const bool trace = getenv("MALUS_GEMM_TRACE") != nullptr;
   if (trace)
-    fprintf(stderr, "malus gemm b%d %dx%dx%d t%d%d -> %s%s tile %dx%d occ %d split %d k_chunk %d\n", batch, M, N, K,
-            transA, transB, dma ? "dma" : "reg", tag, 64 * kTiles[p.ti].tm, 64 * kTiles[p.ti].tn, occupancy(p.ti, v),
-            p.nsplit, p.k_chunk);
+    fprintf(stderr, "malus gemm b%d %dx%dx%d t%d%d -> %s%s tile %dx%d split %d k_chunk %d\n", batch, M, N, K, transA,
+            transB, path, tag, t.bm, t.bn, p.nsplit, p.k_chunk);
 }
 
 // Sum the split-K partials into C (+ D) in split order, then return the
@@ -501,28 +545,26 @@ double launch_dma(const float* A, const float* B, float* C, int batch, int M, in
   // take the plan of the autocast GEMM on f32 copies of them, so the sums
   // run in the same order
   const int v = variant(transA, transB, false, false, true);
-  // a split copy of B (kIoB3) feeds the split product; any other io mask
-  // is bf16 storage, which runs on the bf16 MFMA
-  const bool bf = g_autocast || (L.io & ~kIoB3), x3 = !bf && f32_x3();
-  if ((L.io & kIoB3) && !x3) fail("malus: gemm: a split copy of B needs split f32 products (io mask %d)", L.io);
+  // bf16 storage runs on the bf16 MFMA
+  const bool bf = g_autocast || L.io, x3 = !bf && f32_x3();
   const int vb = (epi ? v | 64 : mapped ? v | 32 : v) | (bf ? kVarBf16 : 0) | (L.io << kVarIoShift) | (x3 ? kVarX3 : 0);
-  const void* fn = kernel_for(0, vb);
-  if (!fn) fail("malus: gemm: no kernel for epilogue %d with transA=%d transB=%d and bf16 storage mask %d", epi, transA,
-                transB, L.io);
+  if (!kernel_for(0, vb))
+    fail("malus: gemm: no kernel for epilogue %d with transA=%d transB=%d and bf16 storage mask %d", epi, transA, transB,
+         L.io);
   if ((L.io & kIoC16) && D) fail("malus: gemm: a bf16 output takes no addend");
-  // Under autocast the GELU GEMM (h = x W1, K = 384, a 3072-workgroup grid
-  // at 128x64) measured 20 % faster on 128x192 tiles.
-  // The GELU forward GEMM takes 128x192 tiles under autocast, and with split
-  // products where that still gives 512 workgroups (C5's 16384 x 1536).
-  const bool gelu_wide = epi == 1 && (bf || (x3 && (long)((M + 127) / 128) * ((N + 191) / 192) * batch >= 512));
-  Plan p = plan_gemm(batch, M, N, K, v | (x3 && epi ? 64 : 0), mapped && L.tri_a, gelu_wide ? 0 : -1, bf, x3);
-  const char* tag = mapped ? " mapped" : "";
-  if ((!split_ok || epi || (L.io & kIoC16)) && p.nsplit > 1) {
-    p.nsplit = 1;
-    p.k_chunk = K;
+  if (epi || (L.io & kIoC16)) split_ok = false;
+  Plan p{-1, 1, K};
+  if (x3 && !(mapped && L.tri_a)) p = plan_x3(batch, M, N, K, split_ok, 1);
+  const bool once = p.ti >= 0;  // each value split once per workgroup
+  if (!once) {
+    // Under autocast the GELU GEMM (h = x W1, K = 384, a 3072-workgroup grid
+    // at 128x64) measured 20 % faster on 128x192 tiles.
+    p = plan_gemm(batch, M, N, K, v, mapped && L.tri_a, epi == 1 && bf ? 0 : -1, bf);
+    if (!split_ok && p.nsplit > 1) p = Plan{p.ti, 1, K};
   }
-  trace_plan(batch, M, N, K, transA, transB, true, p, v, tag);
-  const int bm = 64 * kTiles[p.ti].tm, bn = 64 * kTiles[p.ti].tn;
+  const TileShape ts = tile_shape(once, p.ti);
+  trace_plan(batch, M, N, K, transA, transB, once ? "x3" : "dma", p, ts, mapped ? " mapped" : "");
+  const int bm = ts.bm, bn = ts.bn;
   const int tiles_n = (N + bn - 1) / bn, tiles = ((M + bm - 1) / bm) * tiles_n;
   int nsplit = p.nsplit, k_chunk = p.k_chunk;
   const size_t mn = (size_t)M * N;
@@ -535,8 +577,8 @@ double launch_dma(const float* A, const float* B, float* C, int batch, int M, in
   long split_stride = nsplit > 1 ? (long)mn : 0;
   const float* Dk = nsplit > 1 ? nullptr : D;  // split-K applies the addend in the reduction
   void* args[] = {&A, &B, &dst, &M, &N, &K, &L, &k_chunk, const_cast<int*>(&tiles_n), &split_stride, &Dk, &E};
-  fn = kernel_for(p.ti, vb);
-  MALUS_HIP(hipLaunchKernel(fn, dim3((unsigned)tiles, (unsigned)nsplit, (unsigned)batch), dim3(256), args, 0, s));
+  const void* fn = once ? gemm_x3_kernel(p.ti, vb) : kernel_for(p.ti, vb);
+  MALUS_HIP(hipLaunchKernel(fn, dim3((unsigned)tiles, (unsigned)nsplit, (unsigned)batch), dim3(ts.threads), args, 0, s));
   if (nsplit > 1) split_reduce(dst, C, mn, nsplit, D, s, bucket);
   if (!(mapped && L.tri_a)) return 2.0 * batch * (double)M * N * K;
   double rk = 0;  // sum over tile rows of rows * k range
@@ -572,11 +614,11 @@ void gemm(const float* A, const float* B, float* C, int batch, int M, int N, int
   const long ext_a = (long)(batch - 1) * sA + (long)M * K, ext_b = (long)(batch - 1) * sB + (long)K * N;
   // LDS-DMA path: whole 16-deep K slabs, 16-byte rows, 32-bit byte offsets
   // (a bf16 operand's x-contiguous rows: runs of 8 elements)
-  const int xa = io & kIoA16 ? 8 : 4, xb = io & (kIoB16 | kIoB3) ? 8 : 4;
+  const int xa = io & kIoA16 ? 8 : 4, xb = (io & kIoB16) ? 8 : 4;
   const bool dma = K % 16 == 0 && (transA ? M % xa == 0 : true) && (transB ? true : N % xb == 0) &&
-                   (size_t)ext_a * 4 < (1ull << 31) && (size_t)ext_b * ((io & kIoB3) ? 6 : 4) < (1ull << 31) &&
+                   (size_t)ext_a * 4 < (1ull << 31) && (size_t)ext_b * 4 < (1ull << 31) &&
                    ((size_t)(batch - 1) * sC + (size_t)M * N) * 4 < (1ull << 31) && g_allow_dma;
-  if (io & ~(kIoA16 | kIoB16 | kIoB3)) fail("malus: gemm: bf16 storage mask %d is not an operand mask", io);
+  if (io & ~(kIoA16 | kIoB16)) fail("malus: gemm: bf16 storage mask %d is not an operand mask", io);
   if (dma) {
     GemmLayouts L{dense_layout(lda, sA), dense_layout(ldb, sB), dense_layout(N, sC), (int)ext_a, (int)ext_b};
     L.io = io;
@@ -591,8 +633,9 @@ void gemm(const float* A, const float* B, float* C, int batch, int M, int N, int
   const bool vb = transB ? (K % 4 == 0) : (N % 4 == 0);
   const int v = variant(transA, transB, va, vb, false);
   const Plan p = plan_gemm(batch, M, N, K, v);
-  trace_plan(batch, M, N, K, transA, transB, false, p, v, "");
-  const int bm = 64 * kTiles[p.ti].tm, bn = 64 * kTiles[p.ti].tn;
+  const TileShape ts = tile_shape(false, p.ti);
+  trace_plan(batch, M, N, K, transA, transB, "reg", p, ts, "");
+  const int bm = ts.bm, bn = ts.bn;
   const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + bn - 1) / bn;
   const int tiles = tiles_m * tiles_n;
   int nsplit = p.nsplit, k_chunk = p.k_chunk;
@@ -614,7 +657,7 @@ bool gemm_gelu(const float* A, const float* B, float* C, float* E, int M, int N,
       (backward && !transB))
     return false;
   const long ext_a = (long)M * K, ext_b = (long)K * N;
-  if ((size_t)ext_a * 4 >= (1ull << 31) || (size_t)ext_b * ((io & kIoB3) ? 6 : 4) >= (1ull << 31) ||
+  if ((size_t)ext_a * 4 >= (1ull << 31) || (size_t)ext_b * 4 >= (1ull << 31) ||
       (size_t)M * N * 4 >= (1ull << 31))
     return false;
   GemmLayouts L{dense_layout(K, 0), dense_layout(transB ? K : N, 0), dense_layout(N, 0), (int)ext_a, (int)ext_b};
@@ -633,34 +676,33 @@ bool gemm_grouped(int M, int N, int K, bool transA, bool transB, const GemmLayou
   if (accumulate && !(!transA && transB)) return false;  // built for the projections' dA (NT) only
   GemmLayouts L = Lin;
   const int v = variant(transA, transB, false, false, true);
-  const bool bf = g_autocast || (L.io & ~kIoB3), x3 = !bf && f32_x3();
-  if ((L.io & kIoB3) && !x3) fail("malus: gemm_grouped: a split copy of B needs split f32 products");
-  Plan p = plan_gemm(1, M, N, K, v, false, -1, bf, x3, L.ngroup);
+  const bool bf = g_autocast || L.io, x3 = !bf && f32_x3();
   const bool c_dense = L.c.r.div == 0 && L.c.c.div == 0 && L.c.c.s0 == 1 && L.c.r.s0 == N;
-  if (accumulate || !c_dense || (L.io & kIoC16)) {  // split partials are f32 and dense
-    p.nsplit = 1;
-    p.k_chunk = K;
-  }
-  if (!accumulate && !c_dense && g_forced_tile < 0) {
-    // Separate groups without a split multiply the tile count by ngroup:
-    // take the widest tile that still gives every CU three workgroups (the
-    // q/k/v projections, 16384 x 384 x 384 x 3: 128 x 192 tiles run 9 %
-    // faster than the single GEMM's 128 x 64).
-    for (int ti = 0; ti < kNumTiles; ++ti) {
-      const long tiles = (long)((M + 64 * kTiles[ti].tm - 1) / (64 * kTiles[ti].tm)) *
-                         ((N + 64 * kTiles[ti].tn - 1) / (64 * kTiles[ti].tn)) * L.ngroup;
-      if (N % (64 * kTiles[ti].tn) == 0 && tiles >= 3 * 256) {
-        p.ti = ti;
-        break;
+  const bool split_ok = !accumulate && c_dense && !(L.io & kIoC16);  // split partials are f32 and dense
+  Plan p{-1, 1, K};
+  if (x3) p = plan_x3(1, M, N, K, split_ok, accumulate ? 1 : L.ngroup);
+  const bool once = p.ti >= 0;  // each value split once per workgroup
+  if (!once) {
+    p = plan_gemm(1, M, N, K, v, false, -1, bf);
+    if (!split_ok) p = Plan{p.ti, 1, K};
+    if (!accumulate && !c_dense && g_forced_tile < 0) {
+      // Separate groups without a split multiply the tile count by ngroup:
+      // take the widest tile that still gives every CU three workgroups (the
+      // q/k/v projections, 16384 x 384 x 384 x 3: 128 x 192 tiles run 9 %
+      // faster than the single GEMM's 128 x 64).
+      for (int ti = 0; ti < kNumTiles; ++ti) {
+        const long tiles = (long)((M + 64 * kTiles[ti].tm - 1) / (64 * kTiles[ti].tm)) *
+                           ((N + 64 * kTiles[ti].tn - 1) / (64 * kTiles[ti].tn)) * L.ngroup;
+        if (N % (64 * kTiles[ti].tn) == 0 && tiles >= 3 * 256) {
+          p.ti = ti;
+          break;
+        }
       }
     }
   }
-  static const bool trace = getenv("MALUS_GEMM_TRACE") != nullptr;
-  if (trace)
-    fprintf(stderr, "malus gemm b1 %dx%dx%d t%d%d -> dma grouped%d%s tile %dx%d occ %d split %d k_chunk %d\n", M, N, K,
-            transA, transB, L.ngroup, accumulate ? " acc" : "", 64 * kTiles[p.ti].tm, 64 * kTiles[p.ti].tn,
-            occupancy(p.ti, v), p.nsplit, p.k_chunk);
-  const int bm = 64 * kTiles[p.ti].tm, bn = 64 * kTiles[p.ti].tn;
+  const TileShape ts = tile_shape(once, p.ti);
+  trace_plan(1, M, N, K, transA, transB, once ? "x3" : "dma", p, ts, accumulate ? " grouped acc" : " grouped");
+  const int bm = ts.bm, bn = ts.bn;
   const int tiles_n = (N + bn - 1) / bn, tiles = ((M + bm - 1) / bm) * tiles_n;
   int nsplit = p.nsplit, k_chunk = p.k_chunk;
   const size_t mn = (size_t)M * N;
@@ -678,11 +720,12 @@ bool gemm_grouped(int M, int N, int K, bool transA, bool transB, const GemmLayou
   float* Cp = accumulate ? C : L.gc[0];
   const float *A0 = L.ga[0], *B0 = L.gb[0];
   void* args[] = {&A0, &B0, &Cp, &M, &N, &K, &L, &k_chunk, const_cast<int*>(&tiles_n), &split_stride, &Dk, &E};
-  const void* fn = kernel_for(p.ti, (accumulate ? v | 128 : v | 32) | (bf ? kVarBf16 : 0) | (L.io << kVarIoShift) |
-                                        (x3 ? kVarX3 : 0));
+  const void* fn = once ? gemm_x3_kernel(p.ti, accumulate ? v | 128 : v | 32)
+                        : kernel_for(p.ti, (accumulate ? v | 128 : v | 32) | (bf ? kVarBf16 : 0) |
+                                               (L.io << kVarIoShift) | (x3 ? kVarX3 : 0));
   if (!fn) fail("malus: gemm_grouped: no kernel for transA=%d transB=%d and bf16 storage mask %d", transA, transB, L.io);
-  MALUS_HIP(hipLaunchKernel(fn, dim3((unsigned)tiles, (unsigned)nsplit, accumulate ? 1u : (unsigned)L.ngroup), dim3(256),
-                            args, 0, s));
+  MALUS_HIP(hipLaunchKernel(fn, dim3((unsigned)tiles, (unsigned)nsplit, accumulate ? 1u : (unsigned)L.ngroup),
+                            dim3(ts.threads), args, 0, s));
   if (nsplit > 1) {
     bool vec = mn % 4 == 0;
     for (int g = 0; g < L.ngroup; ++g) vec = vec && (reinterpret_cast<uintptr_t>(outs[g]) & 15) == 0;
@@ -723,7 +766,7 @@ bool mapped_ok(int batch, int M, int N, int K, bool transA, bool transB, const G
   // bytes), of 8 elements for a bf16 operand
   const GemmMap& a_contig = L.a.c;  // A [M][K]: k;  A^T [K][M]: m
   const GemmMap& b_contig = L.b.c;  // B [K][N]: n;  B^T [N][K]: k
-  const int ra = L.io & kIoA16 ? 8 : 4, rb = L.io & (kIoB16 | kIoB3) ? 8 : 4;
+  const int ra = L.io & kIoA16 ? 8 : 4, rb = (L.io & kIoB16) ? 8 : 4;
   if (!map_contig(a_contig, ra) || !map_contig(b_contig, rb)) return false;
   if (transA ? M % ra : 0) return false;
   if (transB ? 0 : N % rb) return false;
@@ -737,7 +780,6 @@ bool mapped_ok(int batch, int M, int N, int K, bool transA, bool transB, const G
   const long eb = map_max(L.b.b, batch) + map_max(L.b.r, transB ? N : K) + map_max(L.b.c, transB ? K : N) + 1;
   const long ec = map_max(L.c.b, batch) + map_max(L.c.r, (M + 127) / 128 * 128) + map_max(L.c.c, N) + 1;
   if (ea > L.ext_a || eb > L.ext_b || L.ext_a >= lim || L.ext_b >= lim || ec >= lim) return false;
-  if ((L.io & kIoB3) && (long)L.ext_b * 6 >= (1l << 31)) return false;  // the three planes' byte offsets
   return true;
 }
 }  // namespace

@@ -58,7 +58,6 @@ const void* io_instance(int v) {
 }  // namespace
 
 const void* gemm_io_kernel(int ti, int v) {
-  if ((v >> 9) & kIoB3) return gemm_io_x3_kernel(ti, v);  // a weight's split copy
   // B in bf16 outside the weight-gradient forms: a weight's bf16 copy
   if (((v >> 9) & kIoB16) && !(v & 8)) return gemm_io_weight_kernel(ti, v);
   switch (ti) {  // the host's tile table: 128x192, 128x128, 128x64, 64x128, 64x64

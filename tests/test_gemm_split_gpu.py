@@ -188,3 +188,44 @@ def test_weight_split_copies_give_the_same_steps(rt):
     assert out[0][0] == out[1][0]
     for i, (u, v) in enumerate(zip(out[0][1], out[1][1])):
         np.testing.assert_array_equal(u, v, err_msg=f"state {i}")
+
+
+@pytest.mark.parametrize("form", ["nn", "nt", "tn"])
+@pytest.mark.parametrize(
+    "m,n,k",
+    [
+        (4, 4, 128),  # one 64x64 tile, almost all of it past the edge; the shortest K of the path
+        (68, 132, 144),  # an odd slab count, a row and a column remainder
+        (1000, 260, 400),
+        (192, 128, 4112),  # split K with an uneven last chunk
+        (2100, 1540, 160),  # 128x128 and wider tiles with remainders on both sides
+        (4100, 3080, 176),
+        (16384, 384, 128),  # 128x192, whole tiles
+        (300, 1028, 8192),
+    ],
+)
+def test_values_split_once_per_workgroup(rt, form, m, n, k):
+    # Each tile and staging form of the kernels that split a value once per
+    # workgroup, against float64: 2^-23 per dropped or rounded piece product
+    # and per f32 addition of a 16-deep slab's six, so the error stays below
+    # (6 k / 16 + k) 2^-24 of the sum of |a b|, and in the norm far below it
+    # (random signs): sqrt(k) 2^-24 of sqrt(k) rms(a) rms(b), times a margin of 4.
+    a = RNG.uniform(-1, 1, (m, k)).astype(np.float32)
+    b = RNG.uniform(-1, 1, (k, n)).astype(np.float32)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    ha = rt.tensor(a if form != "tn" else np.ascontiguousarray(a.T))
+    hb = rt.tensor(b if form != "nt" else np.ascontiguousarray(b.T))
+    like = rt.tensor(np.zeros((m, n), np.float32))
+    with split_mode(rt, True):
+        if form == "nn":
+            out = rt.L.tensor_matmul(ha, hb)
+        elif form == "nt":
+            out = rt.L.malus_std_matmul_bwd_a(like, hb, ha)
+        else:
+            out = rt.L.malus_std_matmul_bwd_b(ha, like, hb)
+        got = rt.numpy(out).astype(np.float64)
+    rt.free(ha, hb, like, out)
+    bound = (6 * k / 16 + k) * 2.0**-24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64))
+    assert np.all(np.abs(got - want) <= bound)
+    rms = np.sqrt(np.mean((got - want) ** 2))
+    assert rms <= 4 * np.sqrt(k) * 2.0**-24 * np.sqrt(np.mean(want**2)), (rms, np.sqrt(np.mean(want**2)))
