@@ -56,7 +56,7 @@ def composed_bwd(q, k, v, p, d, sc):
 
 SHAPES = [(6, 64, 32, 1), (6, 64, 32, 0), (5, 128, 64, 1), (4, 256, 64, 1), (4, 256, 64, 0), (3, 96, 64, 1),
           (2, 512, 64, 1), (1, 1024, 32, 1), (2, 32, 64, 1),
-          (2, 1024, 64, 1), (1, 1024, 64, 0)]  # T >= 1024: the dQ pass runs four query tiles per workgroup
+          (2, 1024, 64, 1), (1, 1024, 64, 0)]
 
 
 @pytest.mark.parametrize("bh,t,hs,causal", SHAPES, ids=[f"bh{a}t{b}hs{c}{'c' if d else 'n'}" for a, b, c, d in SHAPES])
@@ -227,3 +227,46 @@ def test_gpt_flash_steps_deterministic_and_graph_equal(rt):
     assert losses == runs[0][0]
     for a, b in zip(params, runs[0][1]):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("path", ["split", "fp32", "autocast"])
+@pytest.mark.parametrize("causal", [1, 0], ids=["causal", "full"])
+@pytest.mark.parametrize("bh,t,hs", [(3, 32, 32), (2, 64, 64), (3, 96, 32), (2, 160, 64), (1, 416, 64), (1, 544, 32)])
+def test_flash_ragged_wave_groups(rt, bh, t, hs, causal, path):
+    # Sequence lengths that end inside a workgroup's group of 32-row tiles
+    # (two or four of them), against float64.  f32: 1e-5 of the norm, as
+    # above.  Autocast: every product rounds two operands by at most 2^-9 each
+    # (rms 2^-9 / sqrt 3 together about 1.6e-3), the gradients chain three of
+    # them: 1.5e-2 of the norm.
+    q, k, v = (rand(bh, t, hs, lo=-2, hi=2) for _ in range(3))
+    d = rand(bh, t, hs)
+    sc = float(np.float32(1.0 / np.sqrt(hs)))
+    handles = [rt.tensor(a) for a in (q, k, v, d, np.array([[sc]], np.float32))]
+    hq, hk, hv, hd, hsc = handles
+    L = rt.L
+    split, auto = L.malus_gemm_set_f32_split(path != "fp32"), L.malus_autocast(path == "autocast")
+    try:
+        hl, dq, dk, dv = (C.c_int64() for _ in range(4))
+        ho = L.malus_std_flash_attn_fwd(hq, hk, hv, hsc, causal, C.byref(hl))
+        assert L.malus_std_flash_attn_bwd(hd, hq, hk, hv, ho, hl.value, hsc, causal, 0, 0, 0, C.byref(dq), C.byref(dk),
+                                          C.byref(dv)) == 0
+        got = [run(rt, h) for h in (ho, hl.value, dq.value, dk.value, dv.value)]
+    finally:
+        L.malus_gemm_set_f32_split(split)
+        L.malus_autocast(auto)
+    rt.free(*handles)
+    q, k, v, d = (a.astype(np.float64) for a in (q, k, v, d))
+    s = q @ k.transpose(0, 2, 1) * sc
+    if causal:
+        s = np.where(np.triu(np.ones((t, t), bool), 1), -np.inf, s)
+    mx = s.max(2, keepdims=True)
+    e = np.exp(s - mx)
+    p = e / e.sum(2, keepdims=True)
+    dp = d @ v.transpose(0, 2, 1)
+    ds = p * (dp - (dp * p).sum(2, keepdims=True)) * sc
+    want = [p @ v, (mx + np.log(e.sum(2, keepdims=True)))[..., 0], ds @ k, ds.transpose(0, 2, 1) @ q,
+            p.transpose(0, 2, 1) @ d]
+    bar = 1.5e-2 if path == "autocast" else 1e-5
+    for name, g, w in zip(("out", "lse", "dq", "dk", "dv"), got, want):
+        err = np.linalg.norm(g - w) / np.linalg.norm(w)
+        assert err <= bar, (name, err)
