@@ -425,6 +425,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dkv(
   constexpr int NKB = HS / 16, NN = HS / 32, NT = 64 * W;
   using Tl = Tile<HS, NP>;
   __shared__ __attribute__((aligned(1024))) char Qs[2][Tl::SIZE], Os[2][Tl::SIZE];
+  __shared__ __attribute__((aligned(16))) float Ls[2][2][32];  // lse and dsum of the tile's rows
   const int tiles = T / 32;
   const int grp = (int)(blockIdx.x / BH), bh = (int)(blockIdx.x % BH);
   const int lane = threadIdx.x & 63, x = lane & 31, lk = lane >> 5;
@@ -436,8 +437,15 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dkv(
   const float* dOh = head_row(dO, bh, H, T, ldo, HS, 0);
   const int j0 = 32 * kt, key = live ? j0 + x : 0;
   const float sc = scale[0];
-  const float* lseh = lse + (size_t)bh * T;
-  const float* dsh = dsum + (size_t)bh * T;
+  // threads 0 .. 63 stage a tile's row values
+  const float* rowv = (threadIdx.x & 32 ? dsum : lse) + (size_t)bh * T + (threadIdx.x & 31);
+  float rv = 0.0f;
+  auto fetch_rows = [&](int it) {
+    if (threadIdx.x < 64) rv = rowv[32 * it];
+  };
+  auto store_rows = [&](int stage) {
+    if (threadIdx.x < 64) Ls[stage][threadIdx.x >> 5][threadIdx.x & 31] = rv;
+  };
   const int wg_first = CAUSAL ? W * grp : 0;
   const int first = !live ? tiles : CAUSAL ? kt : 0;
 
@@ -445,6 +453,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dkv(
   Stream<HS, NT, false> ost;
   qst.fetch(Qh, HS, wg_first);
   ost.fetch(dOh, ldo, wg_first);
+  fetch_rows(wg_first);
   Frag<NP> kf[NKB], vf[NKB];  // B of S = Q K^T and of dP = dO V^T
 #pragma unroll
   for (int kb = 0; kb < NKB; ++kb) {
@@ -459,29 +468,26 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dkv(
   }
   qst.template store<NP>(Qs[0]);
   ost.template store<NP>(Os[0]);
+  store_rows(0);
   __syncthreads();
   for (int it = wg_first; it < tiles; ++it) {
-    const int cur = (it - wg_first) & 1, i0 = 32 * it;
+    const int cur = (it - wg_first) & 1;
     if (it + 1 < tiles) {
       qst.fetch(Qh, HS, it + 1);
       ost.fetch(dOh, ldo, it + 1);
+      fetch_rows(it + 1);
     }
     if (it >= first) {
-      float Lq[2][8], Dq_[2][8];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        load8(lseh + i0 + 16 * h + 8 * lk, Lq[h]);
-        load8(dsh + i0 + 16 * h + 8 * lk, Dq_[h]);
-      }
       v16f s = v16f{0}, dp = v16f{0};
 #pragma unroll
       for (int kb = 0; kb < NKB; ++kb) {
         s = mul<NP>(Tl::row(Qs[cur], perm_row(x), kb, lk), kf[kb], s);
         dp = mul<NP>(Tl::row(Os[cur], perm_row(x), kb, lk), vf[kb], dp);
+        if (NP == 3 && kb % 2) __builtin_amdgcn_sched_barrier(0);  // hold the fragment reads to what 256 VGPRs take
       }
       // lane = key j0 + x, register r = query i0 + perm_index(r, lk)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = exp_of<NP>(s[r] * sc - Lq[r >> 3][r & 7]);
+      for (int r = 0; r < 16; ++r) s[r] = exp_of<NP>(s[r] * sc - Ls[cur][0][perm_index(r, lk)]);
       if (CAUSAL && it == kt) {
 #pragma unroll
         for (int r = 0; r < 16; ++r)
@@ -489,7 +495,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dkv(
       }
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float diff = dp[r] - Dq_[r >> 3][r & 7];
+        const float diff = dp[r] - Ls[cur][1][perm_index(r, lk)];
         const float dx = s[r] * diff;
         dp[r] = dx * sc;
       }
@@ -506,12 +512,14 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dkv(
         for (int n = 0; n < NN; ++n) {
           dvt[n] = mul<NP>(Tl::col(Os[cur], n, h), p, dvt[n]);
           dkt[n] = mul<NP>(Tl::col(Qs[cur], n, h), ds, dkt[n]);
+          if (NP == 3) __builtin_amdgcn_sched_barrier(0);
         }
       }
     }
     if (it + 1 < tiles) {
       qst.template store<NP>(Qs[cur ^ 1]);
       ost.template store<NP>(Os[cur ^ 1]);
+      store_rows(cur ^ 1);
     }
     __syncthreads();
   }

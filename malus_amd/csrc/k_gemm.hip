@@ -493,6 +493,28 @@ Plan plan_x3(int batch, int M, int N, int K, bool split_ok, int groups) {
   return best;
 }
 
+// ---- bf16 products of f32 operands, rounded once per workgroup (k_gemm_bf.h) ----
+// Tile 0 (256x256) or 1 (256x128), or -1 for the kernels of k_gemm_dma.h.
+// The K split stays the one planned for those, so the sums are the same.
+// A 16-deep slab of a workgroup takes 0.68 us (256x256) or 0.42 us (256x128),
+// its start and end about 4 us, and C goes out at 5 TB/s; measured (256x256 /
+// 256x128 / k_gemm_dma.h): 8192 x 4096 x 1024 125 / 152 / 232 us, 8192 x 1024 x
+// 4096 131 / 111 / 201, 4096^3 178 / 225 / 388, 16384 x 384 x 1536 62 / 48 / 53,
+// 1024 x 4096 x 8192 (A transposed) 122 / 157 / 124.  Those kernels reach 330
+// TFLOP/s, or 550 on the weight gradients' 128x192 tiles, once they fill the
+// chip, which takes far fewer rows.
+int plan_bf(int M, int N, const Plan& p, bool wgrad) {
+  const double slabs = p.k_chunk / BK, out = 4.0 * M * N * p.nsplit / 5e12;
+  auto model = [&](int bn, double slab_us) {
+    const long blocks = (long)((M + 255) / 256) * ((N + bn - 1) / bn) * p.nsplit;
+    return (double)((blocks + 255) / 256) * (slabs * slab_us + 4.0) * 1e-6 + out;
+  };
+  const double wide = model(256, 0.68), half = model(128, 0.42);
+  const double dma = 2.0 * M * N * p.k_chunk * p.nsplit / (wgrad ? 550e12 : 330e12);
+  if (1.1 * (wide < half ? wide : half) >= dma) return -1;
+  return wide < half ? 0 : 1;
+}
+
 // The launch of a plan: the tile's size and threads on either path.
 struct TileShape { int bm, bn; unsigned threads; };
 TileShape tile_shape(bool once, int ti) {
@@ -562,8 +584,10 @@ double launch_dma(const float* A, const float* B, float* C, int batch, int M, in
     p = plan_gemm(batch, M, N, K, v, mapped && L.tri_a, epi == 1 && bf ? 0 : -1, bf);
     if (!split_ok && p.nsplit > 1) p = Plan{p.ti, 1, K};
   }
-  const TileShape ts = tile_shape(once, p.ti);
-  trace_plan(batch, M, N, K, transA, transB, once ? "x3" : "dma", p, ts, mapped ? " mapped" : "");
+  int wide_bf = -1;
+  if (bf && !L.io && !mapped && !epi && batch == 1 && g_forced_tile < 0) wide_bf = plan_bf(M, N, p, transA && K >= 4096);
+  const TileShape ts = wide_bf >= 0 ? TileShape{256, wide_bf ? 128 : 256, 512} : tile_shape(once, p.ti);
+  trace_plan(batch, M, N, K, transA, transB, wide_bf >= 0 ? "bf" : once ? "x3" : "dma", p, ts, mapped ? " mapped" : "");
   const int bm = ts.bm, bn = ts.bn;
   const int tiles_n = (N + bn - 1) / bn, tiles = ((M + bm - 1) / bm) * tiles_n;
   int nsplit = p.nsplit, k_chunk = p.k_chunk;
@@ -577,7 +601,7 @@ double launch_dma(const float* A, const float* B, float* C, int batch, int M, in
   long split_stride = nsplit > 1 ? (long)mn : 0;
   const float* Dk = nsplit > 1 ? nullptr : D;  // split-K applies the addend in the reduction
   void* args[] = {&A, &B, &dst, &M, &N, &K, &L, &k_chunk, const_cast<int*>(&tiles_n), &split_stride, &Dk, &E};
-  const void* fn = once ? gemm_x3_kernel(p.ti, vb) : kernel_for(p.ti, vb);
+  const void* fn = wide_bf >= 0 ? gemm_bf_kernel(wide_bf, vb) : once ? gemm_x3_kernel(p.ti, vb) : kernel_for(p.ti, vb);
   MALUS_HIP(hipLaunchKernel(fn, dim3((unsigned)tiles, (unsigned)nsplit, (unsigned)batch), dim3(ts.threads), args, 0, s));
   if (nsplit > 1) split_reduce(dst, C, mn, nsplit, D, s, bucket);
   if (!(mapped && L.tri_a)) return 2.0 * batch * (double)M * N * K;

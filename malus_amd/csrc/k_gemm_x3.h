@@ -40,7 +40,8 @@ namespace {
 // operands as four 4-byte loads, 64 consecutive rows per wave, with the two
 // 8-byte halves of a chunk dealt to alternate 16-row groups so that the
 // 8-byte stores of a half-wave do not meet in one bank.
-template <int BX, int NT, bool KC>
+// NP: 3 planes, or one of the values rounded to bf16 (k_gemm_bf.h).
+template <int BX, int NT, bool KC, int NP = 3>
 struct X3Stage {
   static constexpr int U = BX * 4 / NT;    // units per thread
   static constexpr int PLANE = BX * 32;    // bytes
@@ -75,7 +76,7 @@ struct X3Stage {
       return __builtin_bit_cast(v4f, v);
     }
   }
-  // splits unit u's values into the three planes at S
+  // splits (rounds) unit u's values into the planes at S
   __device__ __forceinline__ void store(char* S, int u, v4f f) const {
     typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
     unsigned h[2], m[2], l[2];
@@ -83,16 +84,60 @@ struct X3Stage {
     for (int q = 0; q < 2; ++q) {
       const float a = f[2 * q], b = f[2 * q + 1];
       h[q] = pack_bf16(a, b);
-      const float ra = a - bf16_low(h[q]), rb = b - bf16_high(h[q]);
-      m[q] = pack_bf16(ra, rb);
-      l[q] = pack_bf16(ra - bf16_low(m[q]), rb - bf16_high(m[q]));
+      if constexpr (NP == 3) {
+        const float ra = a - bf16_low(h[q]), rb = b - bf16_high(h[q]);
+        m[q] = pack_bf16(ra, rb);
+        l[q] = pack_bf16(ra - bf16_low(m[q]), rb - bf16_high(m[q]));
+      }
     }
     *reinterpret_cast<u32x2*>(S + loff[u]) = u32x2{h[0], h[1]};
-    *reinterpret_cast<u32x2*>(S + PLANE + loff[u]) = u32x2{m[0], m[1]};
-    *reinterpret_cast<u32x2*>(S + 2 * PLANE + loff[u]) = u32x2{l[0], l[1]};
+    if constexpr (NP == 3) {
+      *reinterpret_cast<u32x2*>(S + PLANE + loff[u]) = u32x2{m[0], m[1]};
+      *reinterpret_cast<u32x2*>(S + 2 * PLANE + loff[u]) = u32x2{l[0], l[1]};
+    }
   }
 #endif
 };
+
+// The C elements of a wave's accumulators: register r of (i, j) is C at
+// cn(i, j) + dm(r) * row stride.  f(i, j, live(r), offset(r)) runs once per
+// accumulator; a tile inside C skips the edge tests.
+template <int TM, int TN, bool MAP>
+struct TileOut {
+  const GemmLayout& c;
+  int M, N, m0, n0, li, lk;
+  bool inside;
+  template <class F>
+  __device__ __forceinline__ void for_each(F&& f) const {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int rbase = map_at<MAP>(c.r, m0 + 32 * i) + 4 * lk * c.r.s0;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int n = n0 + 32 * j + li, m = m0 + 32 * i + 4 * lk;
+        const int cn = map_at<MAP>(c.c, n) + rbase;
+        auto off = [&](int r) { return cn + (8 * (r >> 2) + (r & 3)) * c.r.s0; };
+        if (inside) f(i, j, [](int) { return true; }, off);
+        else f(i, j, [&](int r) { return n < N && m + 8 * (r >> 2) + (r & 3) < M; }, off);
+      }
+    }
+  }
+};
+
+template <class Live, class Off>
+__device__ __forceinline__ v16f read16(const float* P, Live&& live, Off&& off) {
+  v16f v = v16f{0};
+#pragma unroll
+  for (int r = 0; r < 16; ++r)
+    if (live(r)) v[r] = P[off(r)];
+  return v;
+}
+template <class Live, class Off>
+__device__ __forceinline__ void write16(float* P, const v16f& v, Live&& live, Off&& off) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r)
+    if (live(r)) P[off(r)] = v[r];
+}
 
 // C = op(A) op(B) (+ D) as k_sgemm_dma computes it with X3 (the same
 // operand maps, epilogues EPI 0..3 and split-K partials); the host
@@ -316,43 +361,14 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN == 4 && (EPI == 3 || TM * TN 
     if (UNR == 4 && s + 2 < nk) body(std::integral_constant<int, 2>{});
   };
 
-  // Element (i, j, r) of the accumulators is C at cn(i, j) + dm(r) * row
-  // stride.  f(i, j, live(r), offset(r)) runs once per accumulator; a tile
-  // inside C skips the edge tests.
-  const bool inside = m0 + BM <= M && n0 + BN <= N;
-  auto for_each = [&](auto&& f) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int rbase = map_at<MAP>(L.c.r, m0 + wm + 32 * i) + 4 * lk * L.c.r.s0;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int n = n0 + wn + 32 * j + li, m = m0 + wm + 32 * i + 4 * lk;
-        const int cn = map_at<MAP>(L.c.c, n) + rbase;
-        auto off = [&](int r) { return cn + (8 * (r >> 2) + (r & 3)) * L.c.r.s0; };
-        if (inside) f(i, j, [](int) { return true; }, off);
-        else f(i, j, [&](int r) { return n < N && m + 8 * (r >> 2) + (r & 3) < M; }, off);
-      }
-    }
-  };
-  auto read = [&](const float* P, auto&& live, auto&& off) {
-    v16f v = v16f{0};
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-      if (live(r)) v[r] = P[off(r)];
-    return v;
-  };
-  auto write = [&](float* P, const v16f& v, auto&& live, auto&& off) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-      if (live(r)) P[off(r)] = v[r];
-  };
+  const TileOut<TM, TN, MAP> out{L.c, M, N, m0 + wm, n0 + wn, li, lk, m0 + BM <= M && n0 + BN <= N};
   if constexpr (EPI == 3) {
     v16f tot[TM][TN];
     for (int g = 0; g < L.ngroup; ++g) {
       run_k(L.ga[g], L.gb[g]);
       if (g == 0) {
-        for_each([&](int i, int j, auto&& live, auto&& off) {
-          tot[i][j] = D ? read(D, live, off) + acc[i][j] : acc[i][j];
+        out.for_each([&](int i, int j, auto&& live, auto&& off) {
+          tot[i][j] = D ? read16(D, live, off) + acc[i][j] : acc[i][j];
         });
       } else {
 #pragma unroll
@@ -361,22 +377,22 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN == 4 && (EPI == 3 || TM * TN 
           for (int j = 0; j < TN; ++j) tot[i][j] = tot[i][j] + acc[i][j];
       }
     }
-    for_each([&](int i, int j, auto&& live, auto&& off) { write(Cf, tot[i][j], live, off); });
+    out.for_each([&](int i, int j, auto&& live, auto&& off) { write16(Cf, tot[i][j], live, off); });
   } else {
     run_k(A, B);
-    for_each([&](int i, int j, auto&& live, auto&& off) {
+    out.for_each([&](int i, int j, auto&& live, auto&& off) {
       v16f v = acc[i][j];
       if constexpr (EPI == 2) {
-        const v16f e = read(Ef, live, off);
+        const v16f e = read16(Ef, live, off);
 #pragma unroll
         for (int r = 0; r < 16; ++r) v[r] = gelu_bwd(e[r], v[r]);
       }
-      if (D) v = read(D, live, off) + v;
-      write(Cf, v, live, off);
+      if (D) v = read16(D, live, off) + v;
+      write16(Cf, v, live, off);
       if constexpr (EPI == 1) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) v[r] = gelu_fwd(v[r]);
-        write(Ef, v, live, off);
+        write16(Ef, v, live, off);
       }
     });
   }

@@ -1,5 +1,6 @@
-// The instances of k_gemm_x3.h, in their own translation unit so the GEMM
-// units build in parallel.
+// The instances of k_gemm_x3.h and k_gemm_bf.h, in their own translation unit
+// so the GEMM units build in parallel.
+#include "k_gemm_bf.h"
 #include "k_gemm_x3.h"
 
 namespace malus {
@@ -32,6 +33,20 @@ const void* gemm_x3_kernel(int tile, int v) {
     case 2: return x3_instance<4, 2, 2, 2, 2>(v);
     default: return x3_instance<2, 2, 1, 1, 4>(v);
   }
+}
+
+template <int WM, int WN, int TM, int TN>
+const void* bf_instance(int v) {
+  const bool ta = v & 8, tb = v & 4;
+  if (ta)
+    return tb ? reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, true, true>)
+              : reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, true, false>);
+  return tb ? reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, false, true>)
+            : reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, false, false>);
+}
+
+const void* gemm_bf_kernel(int tile, int v) {
+  return tile == 0 ? bf_instance<2, 4, 4, 2>(v) : bf_instance<4, 2, 2, 2>(v);
 }
 
 }  // namespace k

@@ -217,3 +217,42 @@ def test_autocast_c4_convergence_parity(rt):
         g.close()
     assert lo < 0.5 * np.log(C4["V"])  # the corpus was learned (4.17 -> about 1.6)
     print(f"autocast C4 100 steps: worst relative loss difference {worst:.2e}")
+
+
+@pytest.mark.parametrize("form", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("m,n,k", [(8192, 1024, 1040), (7940, 2052, 528), (4100, 4092, 400), (516, 4096, 8192)])
+def test_wide_tiles_equal_the_small_ones(rt, form, m, n, k):
+    # The 256-wide tiles that round each value once per workgroup run the
+    # same k slabs in the same order as the kernels they replace, which a
+    # pinned tile selects: the same bits (odd slab counts, remainders in both
+    # dimensions, split K).  The pinned tile's own K split has to be the
+    # planned one, so the split shape is compared by value: f32 sums of k
+    # exact products in another order, 2^-24 sqrt(k) of the norm each, times 4.
+    rng = np.random.default_rng(5)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    b = rng.standard_normal((k, n)).astype(np.float32)
+    ha = rt.tensor(a if form != "tn" else np.ascontiguousarray(a.T))
+    hb = rt.tensor(b if form != "nt" else np.ascontiguousarray(b.T))
+    like = rt.tensor(np.zeros((m, n), np.float32))
+    L = rt.L
+    prev = L.malus_autocast(1)
+    got = []
+    try:
+        for tile in ((0, 0), (2, 1)):
+            assert L.malus_gemm_set_tile(*tile)
+            if form == "nn":
+                out = L.tensor_matmul(ha, hb)
+            elif form == "nt":
+                out = L.malus_std_matmul_bwd_a(like, hb, ha)
+            else:
+                out = L.malus_std_matmul_bwd_b(ha, like, hb)
+            got.append(rt.numpy(out))
+            rt.free(out)
+    finally:
+        L.malus_gemm_set_tile(0, 0)
+        L.malus_autocast(prev)
+    rt.free(ha, hb, like)
+    if k < 1024:
+        np.testing.assert_array_equal(got[0], got[1])
+    d = got[0].astype(np.float64) - got[1]
+    assert np.sqrt(np.mean(d * d)) <= 4 * np.sqrt(k) * 2.0**-24 * np.sqrt(np.mean(got[1].astype(np.float64) ** 2))
