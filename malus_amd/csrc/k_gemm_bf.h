@@ -17,7 +17,7 @@
 // MFMAs of its first 16-deep slab run, the second slab's fragments are read;
 // during the second slab's, the next stage's first fragments (that stage
 // was written a stage ago).  Between the MFMAs the wave rounds and stores
-// stage s + 2 from its staging registers and loads stage s + 3 into them.
+// stage s + 2 from its staging registers and loads stage s + 2 + G into them.
 // The sums run over the k slabs upwards in one MFMA each, as in
 // k_sgemm_dma, so the values are the same for the same K split.
 #pragma once
@@ -31,7 +31,7 @@ namespace {
 // Dense operands (C = op(A) op(B) (+ D) or split-K partials); the host
 // guarantees K % 16 == 0, 16-byte aligned k-contiguous rows and byte offsets
 // below 2^31.  WM x WN waves of TM x TN accumulators.
-template <int WM, int WN, int TM, int TN, bool TA, bool TB>
+template <int WM, int WN, int TM, int TN, bool TA, bool TB, int G>
 __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_bf(const float* __restrict__ A, const float* __restrict__ B,
                                                          float* __restrict__ C, int M, int N, int K, GemmLayouts L,
                                                          int k_chunk, int tiles_n, long split_stride,
@@ -104,13 +104,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_bf(const float* __rest
       }
     }
   };
-  v4f st[2][U];  // a stage's units, slab by slab
-  auto load_unit = [&](int h, int u) {
-    st[h][u] = u < UA ? sa.load(ra, u, dka[h], ksa) : sb.load(rb, u - UA, dkb[h], ksb);
+  v4f st[G][2][U];  // G stages' units, slab by slab
+  auto load_unit = [&](int g, int h, int u) {
+    st[g][h][u] = u < UA ? sa.load(ra, u, dka[h], ksa) : sb.load(rb, u - UA, dkb[h], ksb);
   };
-  auto store_unit = [&](char* S, int h, int u) {
-    if (u < UA) sa.store(S + h * SLAB, u, st[h][u]);
-    else sb.store(S + h * SLAB + PA, u - UA, st[h][u]);
+  auto store_unit = [&](char* S, int g, int h, int u) {
+    if (u < UA) sa.store(S + h * SLAB, u, st[g][h][u]);
+    else sb.store(S + h * SLAB + PA, u - UA, st[g][h][u]);
   };
   auto sync = [&]() {  // this wave's LDS operations are done, then everyone's
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -118,23 +118,27 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_bf(const float* __rest
     asm volatile("" ::: "memory");
   };
   if (nk > 0) {
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {  // stages 0 and 1
+    auto load_stage = [&](int g) {
       next_offsets();
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int u = 0; u < U; ++u) load_unit(h, u);
+        for (int u = 0; u < U; ++u) load_unit(g, h, u);
+    };
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+    for (int s = 0; s < 2; ++s) {  // stages 0 and 1 into LDS
+      load_stage(s % G);
+      if (G == 1 || s == 1) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) store_unit(lds + s * STAGE, h, u);
+        for (int t = G == 1 ? s : 0; t <= s; ++t)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int u = 0; u < U; ++u) store_unit(lds + t * STAGE, t % G, h, u);
+      }
     }
-    next_offsets();
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int u = 0; u < U; ++u) load_unit(h, u);  // stage 2
+    for (int g = 0; g < G; ++g) load_stage(g);  // stages 2 .. 1 + G
     sync();
     bf16x8 fa[2][TM], fb[2][TN];
     auto read = [&](int set, int at) {
@@ -145,13 +149,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_bf(const float* __rest
     };
     read(0, 0);
     int cur = 0, nxt = STAGE, wr = 2 * STAGE;  // LDS offsets of stages s, s + 1 and s + 2
-    auto half = [&](auto hc, int at) {
-      constexpr int H = decltype(hc)::value;
+    auto half = [&](auto gc, auto hc, int at) {
+      constexpr int P = decltype(gc)::value, H = decltype(hc)::value;
       read(H ^ 1, at);  // the next slab's fragments
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        store_unit(lds + wr, H, u);
-        load_unit(H, u);
+        store_unit(lds + wr, P, H, u);
+        load_unit(P, H, u);
       }
 #pragma unroll
       for (int i = 0; i < TM; ++i)
@@ -165,16 +169,20 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_bf(const float* __rest
       }
       __builtin_amdgcn_sched_barrier(0);
     };
-    for (int s = 0; s < nst; ++s) {
+    auto body = [&](auto gc, int s) {
       next_offsets();
-      half(std::integral_constant<int, 0>{}, cur + SLAB);
+      half(gc, std::integral_constant<int, 0>{}, cur + SLAB);
       // an odd slab count: the last stage's second slab repeats the last one
-      if (2 * s + 1 < nk) half(std::integral_constant<int, 1>{}, nxt);
+      if (2 * s + 1 < nk) half(gc, std::integral_constant<int, 1>{}, nxt);
       sync();
       const int t = cur;
       cur = nxt;
       nxt = wr;
       wr = t;
+    };
+    for (int s = 0; s < nst; s += G) {
+      body(std::integral_constant<int, 0>{}, s);
+      if (G == 2 && s + 1 < nst) body(std::integral_constant<int, G - 1>{}, s + 1);
     }
   }
 

@@ -35,18 +35,18 @@ const void* gemm_x3_kernel(int tile, int v) {
   }
 }
 
-template <int WM, int WN, int TM, int TN>
+template <int WM, int WN, int TM, int TN, int G>
 const void* bf_instance(int v) {
   const bool ta = v & 8, tb = v & 4;
   if (ta)
-    return tb ? reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, true, true>)
-              : reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, true, false>);
-  return tb ? reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, false, true>)
-            : reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, false, false>);
+    return tb ? reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, true, true, G>)
+              : reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, true, false, G>);
+  return tb ? reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, false, true, G>)
+            : reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, false, false, G>);
 }
 
 const void* gemm_bf_kernel(int tile, int v) {
-  return tile == 0 ? bf_instance<2, 4, 4, 2>(v) : bf_instance<4, 2, 2, 2>(v);
+  return tile == 0 ? bf_instance<2, 4, 4, 2, 1>(v) : bf_instance<4, 2, 2, 2, 2>(v);
 }
 
 }  // namespace k
