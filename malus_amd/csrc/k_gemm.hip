@@ -455,22 +455,14 @@ constexpr X3Tile kX3Tiles[] = {{128, 192, 256, 2, 1.0, 1.0},
                                {128, 128, 256, 2, 0.66, 0.66},
                                {256, 128, 512, 1, 1.25, 1.25},
                                {64, 64, 256, 4, 0.33, 0.24}};
+constexpr int kX3Count = sizeof(kX3Tiles) / sizeof(kX3Tiles[0]);
+constexpr int kX3K = kX3Count;  // a plan's ti: the waves split K (k_gemm_x3k.h: 32x64 tiles of eight waves)
 
-// The tile and K split with the smallest modelled time of the busiest CU,
-// plus the split-K partials' round trip.  ti < 0: the kernels of
-// k_gemm_dma.h, which keep the batched products (the composed attention's,
-// K = T or the head size), K < 128 (the two slabs in flight are then most of
-// the K loop: 2048 x 512 x 128 takes 7.4 us here and 7.2 there) and the tuning
-// knobs' tiles and splits.
-// groups: the products one grouped launch runs side by side.  They do not
-// change a split, so that a grouped product has the bits of the single one.
-Plan plan_x3(int batch, int M, int N, int K, bool split_ok, int groups) {
-  Plan best{-1, 1, K};
-  read_forced_tile();
-  if (g_forced_tile >= 0 || g_split_target > 0 || batch > 1 || K < 128) return best;
-  if (split_ok) groups = 1;
+// The tile and K split with the smallest modelled time (us) of the busiest
+// CU, plus the split-K partials' round trip.
+double best_x3_tile(int M, int N, int K, bool split_ok, int groups, Plan* best) {
   double best_t = 1e300;
-  for (int ti = 0; ti < (int)(sizeof(kX3Tiles) / sizeof(kX3Tiles[0])); ++ti) {
+  for (int ti = 0; ti < kX3Count; ++ti) {
     const X3Tile& c = kX3Tiles[ti];
     const long tiles = (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * groups;
     for (int per = 0; per <= 3; ++per) {  // no split, or about `per` workgroups per CU
@@ -485,11 +477,35 @@ Plan plan_x3(int batch, int M, int N, int K, bool split_ok, int groups) {
       const long per_cu = (tiles * ns + 255) / 256;
       const long rounds = (per_cu + c.conc - 1) / c.conc;
       // 3 us a round for the first loads and the stores of C
-      double t = 1e-6 * (kc / BK) * (rounds * c.lat + (per_cu - rounds) * c.thr) + rounds * 3e-6;
-      if (ns > 1) t += (ns + 1.0) * M * N * groups * 4.0 / 4e12 + 3e-6;
-      if (t < best_t * 0.999) { best_t = t; best = Plan{ti, ns, kc}; }
+      double t = (kc / BK) * (rounds * c.lat + (per_cu - rounds) * c.thr) + rounds * 3;
+      if (ns > 1) t += (ns + 1.0) * M * N * groups * 4.0 / 4e6 + 3;
+      if (t < best_t * 0.999) { best_t = t; *best = Plan{ti, ns, kc}; }
     }
   }
+  return best_t;
+}
+
+// The plan of a split product; ti < 0: the kernels of k_gemm_dma.h, which
+// keep the batched products (the composed attention's, K = T or the head
+// size), K < 128 (the slabs in flight are then most of the K loop: 2048 x 512 x
+// 128 takes 7.7 us here and 7.2 there) and the tuning knobs' tiles and
+// splits.  groups: the products one grouped launch runs side by side.  They
+// do not change a split, so that a grouped product has the bits of the
+// single one; nor do groups, epilogues or a missing split decide for the
+// kernel whose waves split K, which needs a CU to itself: its 32 x 64 tiles
+// take 0.78 us per 8 slabs (256 x 384 x 384: 12.2 -> 7.5 us, 512^3 15.2 ->
+// 8.5, 128 x 4096 x 1024 18.8 -> 12.4) and lose to a split K from 96 slabs on (256
+// x 384 x 1536 13.0 against 14.4) and in a second round (2048 x 384 x 384,
+// B transposed, 11.8 against 19.6).
+Plan plan_x3(int batch, int M, int N, int K, bool split_ok, int groups) {
+  Plan best{-1, 1, K};
+  read_forced_tile();
+  if (g_forced_tile >= 0 || g_split_target > 0 || batch > 1 || K < 128) return best;
+  if ((long)((M + 31) / 32) * ((N + 63) / 64) <= 256) {
+    const double waves = (K / BK + 7) / 8 * 0.78 + 3.8;
+    if (waves < best_x3_tile(M, N, K, true, 1, &best)) return Plan{kX3K, 1, K};
+  }
+  best_x3_tile(M, N, K, split_ok, split_ok ? 1 : groups, &best);
   return best;
 }
 
@@ -515,9 +531,12 @@ int plan_bf(int M, int N, const Plan& p, bool wgrad) {
   return wide < half ? 0 : 1;
 }
 
+const void* x3_kernel(int ti, int v) { return ti == kX3K ? gemm_x3k_kernel(v) : gemm_x3_kernel(ti, v); }
+
 // The launch of a plan: the tile's size and threads on either path.
 struct TileShape { int bm, bn; unsigned threads; };
 TileShape tile_shape(bool once, int ti) {
+  if (once && ti == kX3K) return TileShape{32, 64, 512};
   if (once) return TileShape{kX3Tiles[ti].bm, kX3Tiles[ti].bn, (unsigned)kX3Tiles[ti].threads};
   return TileShape{64 * kTiles[ti].tm, 64 * kTiles[ti].tn, 256};
 }
@@ -601,8 +620,13 @@ double launch_dma(const float* A, const float* B, float* C, int batch, int M, in
   long split_stride = nsplit > 1 ? (long)mn : 0;
   const float* Dk = nsplit > 1 ? nullptr : D;  // split-K applies the addend in the reduction
   void* args[] = {&A, &B, &dst, &M, &N, &K, &L, &k_chunk, const_cast<int*>(&tiles_n), &split_stride, &Dk, &E};
-  const void* fn = wide_bf >= 0 ? gemm_bf_kernel(wide_bf, vb) : once ? gemm_x3_kernel(p.ti, vb) : kernel_for(p.ti, vb);
-  MALUS_HIP(hipLaunchKernel(fn, dim3((unsigned)tiles, (unsigned)nsplit, (unsigned)batch), dim3(ts.threads), args, 0, s));
+  const void* fn = wide_bf >= 0 ? gemm_bf_kernel(wide_bf, vb) : once ? x3_kernel(p.ti, vb) : kernel_for(p.ti, vb);
+  if (once && p.ti == kX3K) {
+    void* kargs[] = {&A, &B, &C, &M, &N, &K, &L, const_cast<int*>(&tiles_n), &D, &E};
+    MALUS_HIP(hipLaunchKernel(fn, dim3((unsigned)tiles, 1, (unsigned)batch), dim3(ts.threads), kargs, 0, s));
+  } else {
+    MALUS_HIP(hipLaunchKernel(fn, dim3((unsigned)tiles, (unsigned)nsplit, (unsigned)batch), dim3(ts.threads), args, 0, s));
+  }
   if (nsplit > 1) split_reduce(dst, C, mn, nsplit, D, s, bucket);
   if (!(mapped && L.tri_a)) return 2.0 * batch * (double)M * N * K;
   double rk = 0;  // sum over tile rows of rows * k range
@@ -744,12 +768,13 @@ bool gemm_grouped(int M, int N, int K, bool transA, bool transB, const GemmLayou
   float* Cp = accumulate ? C : L.gc[0];
   const float *A0 = L.ga[0], *B0 = L.gb[0];
   void* args[] = {&A0, &B0, &Cp, &M, &N, &K, &L, &k_chunk, const_cast<int*>(&tiles_n), &split_stride, &Dk, &E};
-  const void* fn = once ? gemm_x3_kernel(p.ti, accumulate ? v | 128 : v | 32)
+  const void* fn = once ? x3_kernel(p.ti, accumulate ? v | 128 : v | 32)
                         : kernel_for(p.ti, (accumulate ? v | 128 : v | 32) | (bf ? kVarBf16 : 0) |
                                                (L.io << kVarIoShift) | (x3 ? kVarX3 : 0));
   if (!fn) fail("malus: gemm_grouped: no kernel for transA=%d transB=%d and bf16 storage mask %d", transA, transB, L.io);
+  void* kargs[] = {&A0, &B0, &Cp, &M, &N, &K, &L, const_cast<int*>(&tiles_n), &Dk, &E};
   MALUS_HIP(hipLaunchKernel(fn, dim3((unsigned)tiles, (unsigned)nsplit, accumulate ? 1u : (unsigned)L.ngroup),
-                            dim3(ts.threads), args, 0, s));
+                            dim3(ts.threads), once && p.ti == kX3K ? kargs : args, 0, s));
   if (nsplit > 1) {
     bool vec = mn % 4 == 0;
     for (int g = 0; g < L.ngroup; ++g) vec = vec && (reinterpret_cast<uintptr_t>(outs[g]) & 15) == 0;

@@ -19,6 +19,8 @@ const void* gemm_io_weight_kernel(int ti, int v);
 // The split-product instances that split each operand value once per
 // workgroup (k_gemm_x3.h), for tile index `tile` of the host's table.
 const void* gemm_x3_kernel(int tile, int v);
+// The split-product instances whose waves split K (k_gemm_x3k.h).
+const void* gemm_x3k_kernel(int v);
 // The bf16 instances that round each operand value once per workgroup
 // (k_gemm_bf.h; dense operands): tile 0 = 256x256, 1 = 256x128.
 const void* gemm_bf_kernel(int tile, int v);

@@ -194,8 +194,10 @@ def test_weight_split_copies_give_the_same_steps(rt):
 @pytest.mark.parametrize(
     "m,n,k",
     [
-        (4, 4, 128),  # one 64x64 tile, almost all of it past the edge; the shortest K of the path
+        (4, 4, 128),  # one tile, almost all of it past the edge; the shortest K of the path
         (68, 132, 144),  # an odd slab count, a row and a column remainder
+        (36, 64, 912),  # the waves' K ranges of unequal length
+        (260, 1000, 1024),
         (1000, 260, 400),
         (192, 128, 4112),  # split K with an uneven last chunk
         (2100, 1540, 160),  # 128x128 and wider tiles with remainders on both sides
