@@ -35,6 +35,10 @@ namespace malus { struct TensorBuffer; }
 int64_t matmul_impl(int64_t a, int64_t b, const malus::TensorBuffer* D);
 int64_t matmul_bwd_a_impl(int64_t a, int64_t b, int64_t dout, const malus::TensorBuffer* D);
 int64_t matmul_bwd_b_impl(int64_t a, int64_t b, int64_t dout, const malus::TensorBuffer* D);
+// old + dout * other for a multiply's VJP whose target already has the
+// gradient `old` (the product, then GradAcc's add, in one pass); 0 unless all three
+// are f32 tensors of the target's shape.
+int64_t mul_bwd_acc(int64_t dout, int64_t other, int64_t target, const malus::TensorBuffer* old);
 int64_t layernorm_bwd_impl(int64_t y, int64_t var, int64_t dout, int64_t axis, const malus::TensorBuffer* D);
 // out = layernorm(x, axis=-1) * w in one kernel, and the VJP for x (the
 // layernorm VJP of dout * w, + D); the VJP for w is malus_std_mul_bwd_b(dout, y, w).

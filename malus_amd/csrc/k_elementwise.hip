@@ -109,6 +109,19 @@ __global__ __launch_bounds__(kBlock) void k_binary_same(const float* __restrict_
           [&](size_t i) { return binop<OP>(p[i], q[i]); });
 }
 
+// old + p * q, the product rounded before the add: a multiply's VJP with the
+// gradient accumulation folded in (16 B per element instead of the product's 12
+// and the sum's 12; 2^26 elements: 252 -> 168 us).
+__global__ __launch_bounds__(kBlock) void k_mul_add(const float* __restrict__ p, const float* __restrict__ q,
+                                                    const float* __restrict__ old, float* __restrict__ out, size_t n) {
+  ew_loop(n, out,
+          [&](size_t i) {
+            float4 a = ld4(p, i), b = ld4(q, i), c = ld4(old, i);
+            return make_float4(c.x + a.x * b.x, c.y + a.y * b.y, c.z + a.z * b.z, c.w + a.w * b.w);
+          },
+          [&](size_t i) { return old[i] + p[i] * q[i]; });
+}
+
 // q broadcast along leading dims: q index = i % qn (qn % 4 == 0 for the float4 path).
 template <int OP>
 __global__ __launch_bounds__(kBlock) void k_binary_rowb(const float* __restrict__ p, const float* __restrict__ q,
@@ -293,6 +306,12 @@ void binary_same(int op, const float* p, const float* q, float* out, size_t n, h
   if (!n) return;
   dispatch_binop(op, [&](auto o) { k_binary_same<decltype(o)::value><<<ew_grid(n / 4 + 1), kBlock, 0, s>>>(p, q, out, n); });
   post_launch("binary_same");
+}
+
+void mul_add(const float* p, const float* q, const float* old, float* out, size_t n, hipStream_t s) {
+  if (!n) return;
+  k_mul_add<<<ew_grid(n / 4 + 1), kBlock, 0, s>>>(p, q, old, out, n);
+  post_launch("mul_add");
 }
 
 void binary_rowbcast(int op, const float* p, const float* q, float* out, size_t n, size_t qn, hipStream_t s) {

@@ -505,6 +505,19 @@ int64_t malus_std_sub_bwd_b(int64_t dout, int64_t b) {
   return r;
   API_CATCH(0)
 }
+}  // extern "C"
+
+int64_t mul_bwd_acc(int64_t dout, int64_t other, int64_t target, const TensorBuffer* old) {
+  const TensorBuffer *d = T(dout), *o = T(other), *t = T(target);
+  for (const TensorBuffer* x : {d, o, old})
+    if (x->dtype != F32 || !same_shape(x, t)) return 0;
+  TensorBuffer* out = alloc_tensor(F32, t->shape, t->ndim);
+  k::mul_add(d->f32(), o->f32(), old->f32(), out->f32(), out->len, stream());
+  return done(out, "mul_bwd_acc");
+}
+
+extern "C" {
+
 int64_t malus_std_mul_bwd_a(int64_t dout, int64_t a, int64_t b) {
   API_TRY
   if (same_shape(T(dout), T(b)) && !same_shape(T(dout), T(a)))  // reduce dout * b without materializing it

@@ -705,8 +705,20 @@ void backward(int64_t loss) {
         int32_t sa = n.op == Mul ? MulBwdA : DivBwdA, sb = n.op == Mul ? MulBwdB : DivBwdB;
         if (na) need_values(b);
         if (nb) { need_values(a); need_values(b); }
-        if (na) accumulate(grads, a, slot_fn<Fn3>(sa)(dout, a, b));
-        if (nb) accumulate(grads, b, slot_fn<Fn3>(sb)(dout, a, b));
+        // a product's gradient folds into an existing one in the same pass
+        auto folded = [&](int64_t x, int64_t other, bool own) {
+          auto g = grads.find(x);
+          if (!own || n.op != Mul || g == grads.end() || !slot_is(GradAcc, &malus_std_broadcast_add_fwd)) return false;
+          const int64_t r = mul_bwd_acc(dout, other, x, T(g->second));
+          if (!r) return false;
+          release(T(g->second));
+          g->second = r;
+          return true;
+        };
+        if (na && !folded(a, b, slot_is(MulBwdA, &malus_std_mul_bwd_a)))
+          accumulate(grads, a, slot_fn<Fn3>(sa)(dout, a, b));
+        if (nb && !folded(b, a, slot_is(MulBwdB, &malus_std_mul_bwd_b)))
+          accumulate(grads, b, slot_fn<Fn3>(sb)(dout, a, b));
         break;
       }
       case Sigmoid: accumulate(grads, n.saved[0], slot_fn<Fn2>(SigmoidBwd)(n.output, dout)); break;

@@ -225,3 +225,33 @@ def test_c5_three_step_trajectory(rt):
     finally:
         rt.L.malus_gpt_free(g)
         rt.L.tape_reset()
+
+
+@pytest.mark.parametrize("shape_b", [(37, 259), (1, 259), (259,)], ids=["same", "row", "rank1"])
+def test_multiply_gradients_fold_into_existing_ones(tape, shape_b):
+    # z = a*b*a - a*b + a: products whose operands already have a gradient,
+    # of the product's shape (one pass: old + dout * other) and broadcast (the
+    # general path).  With the fused VJPs off every step runs by itself; the
+    # product is rounded before the add either way, so the bits are the same.
+    rt = tape
+    rng = np.random.default_rng(8)
+    a, b = rng.standard_normal((37, 259)).astype(np.float32), rng.standard_normal(shape_b).astype(np.float32)
+    got = []
+    for fused in (1, 0):
+        rt.L.malus_tape_set_fused_vjps(fused)
+        try:
+            ha, hb = leaf(rt, a), leaf(rt, b)
+            rec = lambda op, f, x, y: (lambda h: (rt.L.tape_record_binop(OP[op], x, y, h), h)[1])(  # noqa: E731
+                rt.L.malus_std_broadcast_fwd(f, x, y))
+            ab = rec("Mul", M.MUL, ha, hb)
+            aba = rec("Mul", M.MUL, ab, ha)
+            s = rec("Sub", M.SUB, aba, ab)
+            z = rec("Add", M.ADD, s, ha)
+            rt.L.backward(z)
+            got.append([grad(rt, ha), grad(rt, hb)])
+            rt.free(ha, hb, ab, aba, s, z)
+            rt.L.tape_reset()
+        finally:
+            rt.L.malus_tape_set_fused_vjps(1)
+    for f, u in zip(*got):
+        assert_bitexact(f, u, "folded gradients")
