@@ -1,9 +1,11 @@
 // Row kernels: softmax, layernorm, cross-entropy (forward and VJP).
-// Contiguous rows (inner == 1) up to 4096 wide run one wave64 per row with
+// Contiguous rows (inner == 1) up to 2048 wide run one wave64 per row with
 // the whole row held in registers: one HBM read per input element and one
-// write per output element, reductions by wave shuffles.  Other shapes
-// (reductions over a non-last axis, rows wider than 4096) use a sequential
-// per-(outer, inner) kernel that follows the reference loops directly.
+// write per output element, reductions by wave shuffles.  Rows up to 16384
+// wide run the same kernels with the row spread over a workgroup of W = 256,
+// 512 or 1024 threads (16 values each), whose waves' sums meet in LDS.  Other shapes (reductions over a non-last
+// axis, wider rows) use a sequential per-(outer, inner) kernel that follows
+// the reference loops directly.
 #include "common.h"
 
 namespace malus {
@@ -25,23 +27,52 @@ __device__ __forceinline__ float wmax(float v) {
   return v;
 }
 
+// The row of a wave (W = 64) or a workgroup (W threads), and sums and maxima
+// over it; red: one float per wave, not reused by the kernel.
+template <int W>
+__device__ __forceinline__ size_t row_index() {
+  return W == kWave ? (size_t)blockIdx.x * kRowsPerBlock + threadIdx.x / kWave : (size_t)blockIdx.x;
+}
+template <int W>
+__device__ __forceinline__ float rsum(float v, float* red) {
+  v = wsum(v);
+  if (W == kWave) return v;
+  if (threadIdx.x % kWave == 0) red[threadIdx.x / kWave] = v;
+  __syncthreads();
+  v = red[0];
+#pragma unroll
+  for (int i = 1; i < W / kWave; ++i) v += red[i];
+  return v;
+}
+template <int W>
+__device__ __forceinline__ float rmax(float v, float* red) {
+  v = wmax(v);
+  if (W == kWave) return v;
+  if (threadIdx.x % kWave == 0) red[threadIdx.x / kWave] = v;
+  __syncthreads();
+  v = red[0];
+#pragma unroll
+  for (int i = 1; i < W / kWave; ++i) v = fmaxf(v, red[i]);
+  return v;
+}
+
 // Register tile of one row: NV float4 chunks per lane.  Element e of the
 // lane's tile is column col(e).  VM: 0 scalar, 1 float4, 2 float4 with
 // non-temporal loads (for operands too large to stay in the 256 MB
-// last-level cache between kernels).  VEC: chunk j covers columns 4*(lane+64j)..+3;
-// scalar: element e is column lane + 64*e.
-template <int NV, int VM>
+// last-level cache between kernels).  VEC: chunk j covers columns 4*(lane+W*j)..+3;
+// scalar: element e is column lane + W*e.
+template <int NV, int VM, int W = kWave>
 struct RowTile {
   static constexpr bool VEC = VM > 0, NT = VM == 2;
   float v[NV * 4];
   __device__ __forceinline__ static uint32_t col(int e, int lane) {
-    return VEC ? 4u * (uint32_t)(lane + kWave * (e / 4)) + (uint32_t)(e % 4) : (uint32_t)(lane + kWave * e);
+    return VEC ? 4u * (uint32_t)(lane + W * (e / 4)) + (uint32_t)(e % 4) : (uint32_t)(lane + W * e);
   }
   __device__ __forceinline__ void load(const float* __restrict__ row, uint32_t axis, int lane, float pad) {
     if (VEC) {
 #pragma unroll
       for (int j = 0; j < NV; ++j) {
-        uint32_t c4 = (uint32_t)(lane + kWave * j);
+        uint32_t c4 = (uint32_t)(lane + W * j);
         if (4 * c4 < axis) {
           const v4f t = NT ? __builtin_nontemporal_load(reinterpret_cast<const v4f*>(row) + c4)
                            : reinterpret_cast<const v4f*>(row)[c4];
@@ -62,7 +93,7 @@ struct RowTile {
     if (VEC) {
 #pragma unroll
       for (int j = 0; j < NV; ++j) {
-        uint32_t c4 = (uint32_t)(lane + kWave * j);
+        uint32_t c4 = (uint32_t)(lane + W * j);
         // ordinary store: the next op (often a GEMM) reads this row back from cache
         if (4 * c4 < axis) reinterpret_cast<float4*>(row)[c4] = make_float4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
       }
@@ -78,18 +109,19 @@ struct RowTile {
 };
 
 // softmax_axis_cpu (metal.rs:1439-1467): m = max, e = exp(x - m), s = sum e, y = e / s
-template <int NV, int VM>
-__global__ __launch_bounds__(256) void k_softmax_rows(const float* __restrict__ x, float* __restrict__ y, size_t rows,
+template <int NV, int VM, int W>
+__global__ __launch_bounds__(W == kWave ? 256 : W) void k_softmax_rows(const float* __restrict__ x, float* __restrict__ y, size_t rows,
                                                       uint32_t axis) {
-  const size_t row = (size_t)blockIdx.x * kRowsPerBlock + threadIdx.x / kWave;
-  const int lane = threadIdx.x % kWave;
+  __shared__ float red[2][W / kWave];
+  const size_t row = row_index<W>();
+  const int lane = threadIdx.x % W;
   if (row >= rows) return;
-  RowTile<NV, VM> t;
+  RowTile<NV, VM, W> t;
   t.load(x + row * axis, axis, lane, -INFINITY);
   float m = -INFINITY;
 #pragma unroll
   for (int e = 0; e < NV * 4; ++e) m = fmaxf(m, t.v[e]);
-  m = wmax(m);
+  m = rmax<W>(m, red[0]);
   float s = 0.0f;
 #pragma unroll
   for (int e = 0; e < NV * 4; ++e) {
@@ -97,7 +129,7 @@ __global__ __launch_bounds__(256) void k_softmax_rows(const float* __restrict__ 
     t.v[e] = ex;
     s += ex;
   }
-  s = wsum(s);
+  s = rsum<W>(s, red[1]);
 #pragma unroll
   for (int e = 0; e < NV * 4; ++e) t.v[e] = t.v[e] / s;
   t.store(y + row * axis, axis, lane);
@@ -107,15 +139,16 @@ __global__ __launch_bounds__(256) void k_softmax_rows(const float* __restrict__ 
 // the row, fusing nanogpt_modular.ml's `scores * scale`, `+ mask` and
 // softmax.  Each op rounds like its own kernel (the product, then the sum,
 // then softmax_axis_cpu), so y equals the three-kernel result bit for bit.
-template <int NV, int VM>
-__global__ __launch_bounds__(256) void k_scale_mask_softmax_rows(const float* __restrict__ x, const float* __restrict__ scale,
+template <int NV, int VM, int W>
+__global__ __launch_bounds__(W == kWave ? 256 : W) void k_scale_mask_softmax_rows(const float* __restrict__ x, const float* __restrict__ scale,
                                                                  const float* __restrict__ mask, float* __restrict__ y,
                                                                  size_t rows, uint32_t axis, uint32_t mask_rows) {
-  const size_t row = (size_t)blockIdx.x * kRowsPerBlock + threadIdx.x / kWave;
-  const int lane = threadIdx.x % kWave;
+  __shared__ float red[2][W / kWave];
+  const size_t row = row_index<W>();
+  const int lane = threadIdx.x % W;
   if (row >= rows) return;
   const float sc = scale[0];
-  RowTile<NV, VM> t, mk;
+  RowTile<NV, VM, W> t, mk;
   t.load(x + row * axis, axis, lane, 0.0f);
   mk.load(mask + (row % mask_rows) * axis, axis, lane, 0.0f);
 #pragma unroll
@@ -126,7 +159,7 @@ __global__ __launch_bounds__(256) void k_scale_mask_softmax_rows(const float* __
   float m = -INFINITY;
 #pragma unroll
   for (int e = 0; e < NV * 4; ++e) m = fmaxf(m, t.v[e]);
-  m = wmax(m);
+  m = rmax<W>(m, red[0]);
   float s = 0.0f;
 #pragma unroll
   for (int e = 0; e < NV * 4; ++e) {
@@ -134,26 +167,27 @@ __global__ __launch_bounds__(256) void k_scale_mask_softmax_rows(const float* __
     t.v[e] = ex;
     s += ex;
   }
-  s = wsum(s);
+  s = rsum<W>(s, red[1]);
 #pragma unroll
   for (int e = 0; e < NV * 4; ++e) t.v[e] = t.v[e] / s;
   t.store(y + row * axis, axis, lane);
 }
 
 // tape.rs:1150-1161: dx = s * (dout - sum(dout * s))
-template <int NV, int VM>
-__global__ __launch_bounds__(256) void k_softmax_bwd_rows(const float* __restrict__ y, const float* __restrict__ dout,
+template <int NV, int VM, int W>
+__global__ __launch_bounds__(W == kWave ? 256 : W) void k_softmax_bwd_rows(const float* __restrict__ y, const float* __restrict__ dout,
                                                           float* __restrict__ dx, size_t rows, uint32_t axis) {
-  const size_t row = (size_t)blockIdx.x * kRowsPerBlock + threadIdx.x / kWave;
-  const int lane = threadIdx.x % kWave;
+  __shared__ float red[1][W / kWave];
+  const size_t row = row_index<W>();
+  const int lane = threadIdx.x % W;
   if (row >= rows) return;
-  RowTile<NV, VM> s, d;
+  RowTile<NV, VM, W> s, d;
   s.load(y + row * axis, axis, lane, 0.0f);
   d.load(dout + row * axis, axis, lane, 0.0f);
   float acc = 0.0f;
 #pragma unroll
   for (int e = 0; e < NV * 4; ++e) { float p = d.v[e] * s.v[e]; acc += p; }
-  acc = wsum(acc);
+  acc = rsum<W>(acc, red[0]);
 #pragma unroll
   for (int e = 0; e < NV * 4; ++e) { float diff = d.v[e] - acc; s.v[e] = s.v[e] * diff; }
   s.store(dx + row * axis, axis, lane);
@@ -162,26 +196,27 @@ __global__ __launch_bounds__(256) void k_softmax_bwd_rows(const float* __restric
 // tensor_layernorm_axis (metal.rs:1486-1533): y = (x - mu) / sqrt(var + eps)
 // With w: also out = y * w[col] (the `layernorm(x) * w` of nanogpt_modular.ml:47,
 // rounded like the separate broadcast multiply).
-template <int NV, int VM>
-__global__ __launch_bounds__(256) void k_layernorm_rows(const float* __restrict__ x, float* __restrict__ y,
+template <int NV, int VM, int W>
+__global__ __launch_bounds__(W == kWave ? 256 : W) void k_layernorm_rows(const float* __restrict__ x, float* __restrict__ y,
                                                         float* __restrict__ var, size_t rows, uint32_t axis, float eps,
                                                         const float* __restrict__ w, float* __restrict__ out) {
-  const size_t row = (size_t)blockIdx.x * kRowsPerBlock + threadIdx.x / kWave;
-  const int lane = threadIdx.x % kWave;
+  __shared__ float red[2][W / kWave];
+  const size_t row = row_index<W>();
+  const int lane = threadIdx.x % W;
   if (row >= rows) return;
-  RowTile<NV, VM> t;
+  RowTile<NV, VM, W> t;
   t.load(x + row * axis, axis, lane, 0.0f);
   float s = 0.0f;
 #pragma unroll
   for (int e = 0; e < NV * 4; ++e) s += t.v[e];
-  s = wsum(s);
+  s = rsum<W>(s, red[0]);
   const float mu = s / (float)axis;
   float q = 0.0f;
 #pragma unroll
   for (int e = 0; e < NV * 4; ++e) {
     if (t.valid(e, lane, axis)) { float dd = t.v[e] - mu; q += dd * dd; }
   }
-  q = wsum(q);
+  q = rsum<W>(q, red[1]);
   const float va = q / (float)axis;
   const float sigma = sqrtf(va + eps);
 #pragma unroll
@@ -189,7 +224,7 @@ __global__ __launch_bounds__(256) void k_layernorm_rows(const float* __restrict_
   t.store(y + row * axis, axis, lane);
   if (lane == 0 && var) var[row] = va;
   if (w) {
-    RowTile<NV, VM == 2 ? 1 : VM> wt;  // w is re-read by every row: cached loads
+    RowTile<NV, VM == 2 ? 1 : VM, W> wt;  // w is re-read by every row: cached loads
     wt.load(w, axis, lane, 0.0f);
 #pragma unroll
     for (int e = 0; e < NV * 4; ++e) t.v[e] = t.v[e] * wt.v[e];
@@ -198,20 +233,21 @@ __global__ __launch_bounds__(256) void k_layernorm_rows(const float* __restrict_
 }
 
 // tape.rs:1162-1186: dx = ((dy - mean(dy)) - y * mean(dy*y)) * (1 / sqrt(var + eps))
-template <int NV, int VM>
-__global__ __launch_bounds__(256) void k_layernorm_bwd_rows(const float* __restrict__ y, const float* __restrict__ var,
+template <int NV, int VM, int W>
+__global__ __launch_bounds__(W == kWave ? 256 : W) void k_layernorm_bwd_rows(const float* __restrict__ y, const float* __restrict__ var,
                                                             const float* __restrict__ dout, float* __restrict__ dx,
                                                             size_t rows, uint32_t axis, float eps,
                                                             const float* __restrict__ addend,
                                                             const float* __restrict__ w) {
-  const size_t row = (size_t)blockIdx.x * kRowsPerBlock + threadIdx.x / kWave;
-  const int lane = threadIdx.x % kWave;
+  __shared__ float red[2][W / kWave];
+  const size_t row = row_index<W>();
+  const int lane = threadIdx.x % W;
   if (row >= rows) return;
-  RowTile<NV, VM> yt, dt;
+  RowTile<NV, VM, W> yt, dt;
   yt.load(y + row * axis, axis, lane, 0.0f);
   dt.load(dout + row * axis, axis, lane, 0.0f);
   if (w) {  // dout is the gradient of y * w: dy = dout * w, rounded like the multiply's VJP
-    RowTile<NV, VM == 2 ? 1 : VM> wt;
+    RowTile<NV, VM == 2 ? 1 : VM, W> wt;
     wt.load(w, axis, lane, 0.0f);
 #pragma unroll
     for (int e = 0; e < NV * 4; ++e) dt.v[e] = dt.v[e] * wt.v[e];
@@ -219,8 +255,8 @@ __global__ __launch_bounds__(256) void k_layernorm_bwd_rows(const float* __restr
   float s1 = 0.0f, s2 = 0.0f;
 #pragma unroll
   for (int e = 0; e < NV * 4; ++e) { s1 += dt.v[e]; float p = dt.v[e] * yt.v[e]; s2 += p; }
-  s1 = wsum(s1);
-  s2 = wsum(s2);
+  s1 = rsum<W>(s1, red[0]);
+  s2 = rsum<W>(s2, red[1]);
   const float dy_mean = s1 / (float)axis;
   const float dyy_mean = s2 / (float)axis;
   const float inv_sigma = 1.0f / sqrtf(var[row] + eps);
@@ -450,20 +486,21 @@ __global__ __launch_bounds__(256) void k_layernorm_bwd_scale_rows32(const float*
 
 // cross_entropy.ml:18-28 / metal.rs:1555-1598: probs = softmax(logits, 1),
 // nll[i] = -log(probs[i, t_i]) read back from the rounded probability.
-template <int NV, int VM>
-__global__ __launch_bounds__(256) void k_ce_fwd_rows(const float* __restrict__ logits, const int32_t* __restrict__ tgt,
+template <int NV, int VM, int W>
+__global__ __launch_bounds__(W == kWave ? 256 : W) void k_ce_fwd_rows(const float* __restrict__ logits, const int32_t* __restrict__ tgt,
                                                      float* __restrict__ probs, float* __restrict__ nll, size_t rows,
                                                      uint32_t axis, int32_t* __restrict__ err) {
-  const size_t row = (size_t)blockIdx.x * kRowsPerBlock + threadIdx.x / kWave;
-  const int lane = threadIdx.x % kWave;
+  __shared__ float red[2][W / kWave];
+  const size_t row = row_index<W>();
+  const int lane = threadIdx.x % W;
   if (row >= rows) return;
   const int32_t tg = tgt[row];  // issued with the row's loads
-  RowTile<NV, VM> t;
+  RowTile<NV, VM, W> t;
   t.load(logits + row * axis, axis, lane, -INFINITY);
   float m = -INFINITY;
 #pragma unroll
   for (int e = 0; e < NV * 4; ++e) m = fmaxf(m, t.v[e]);
-  m = wmax(m);
+  m = rmax<W>(m, red[0]);
   float s = 0.0f;
 #pragma unroll
   for (int e = 0; e < NV * 4; ++e) {
@@ -471,7 +508,7 @@ __global__ __launch_bounds__(256) void k_ce_fwd_rows(const float* __restrict__ l
     t.v[e] = ex;
     s += ex;
   }
-  s = wsum(s);
+  s = rsum<W>(s, red[1]);
 #pragma unroll
   for (int e = 0; e < NV * 4; ++e) t.v[e] = t.v[e] / s;
   t.store(probs + row * axis, axis, lane);
@@ -503,23 +540,35 @@ __global__ __launch_bounds__(256) void k_ce_bwd(const float* __restrict__ probs,
   }
 }
 
-// Same expression, four consecutive columns of one row per thread (v % 4 == 0,
-// fewer than 2^32 elements): 32-bit index math, non-temporal streaming.
+// Same expression, four consecutive elements per thread (v >= 4, fewer than
+// 2^32 elements): 32-bit index math, non-temporal streaming (against the
+// scalar form's 64-bit division per element, 65536 x 1023 forward + backward
+// 233 -> 174 us).  WHOLE: v % 4 == 0, so the four are in one row; otherwise
+// the last of them may be the first of the next row, and the total's
+// remainder goes element by element.
+template <bool WHOLE>
 __global__ __launch_bounds__(256) void k_ce_bwd4(const float* __restrict__ probs, const int32_t* __restrict__ tgt,
                                                  const float* __restrict__ dout, float scale_host, float* __restrict__ dx,
-                                                 uint32_t n, uint32_t v, uint32_t total4) {
+                                                 uint32_t n, uint32_t v, uint32_t total) {
   const float scale = dout ? dout[0] / (float)n : scale_host;
-  const uint32_t stride = gridDim.x * blockDim.x;
-  for (uint32_t f4 = blockIdx.x * blockDim.x + threadIdx.x; f4 < total4; f4 += stride) {
+  const uint32_t stride = gridDim.x * blockDim.x, id = blockIdx.x * blockDim.x + threadIdx.x, total4 = total / 4;
+  for (uint32_t f4 = id; f4 < total4; f4 += stride) {
     const uint32_t f = 4 * f4, i = f / v, j = f - i * v;
-    const int32_t t = tgt[i];
-    const v4f p = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(probs) + f4);
-    float g0 = p.x, g1 = p.y, g2 = p.z, g3 = p.w;
-    if ((int32_t)j == t) g0 = g0 - 1.0f;
-    if ((int32_t)(j + 1) == t) g1 = g1 - 1.0f;
-    if ((int32_t)(j + 2) == t) g2 = g2 - 1.0f;
-    if ((int32_t)(j + 3) == t) g3 = g3 - 1.0f;
-    __builtin_nontemporal_store(v4f{g0 * scale, g1 * scale, g2 * scale, g3 * scale}, reinterpret_cast<v4f*>(dx) + f4);
+    const int32_t t = tgt[i], u = WHOLE ? 0 : tgt[i + 1 < n ? i + 1 : i];
+    v4f g = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(probs) + f4);
+#pragma unroll
+    for (uint32_t c = 0; c < 4; ++c) {
+      const uint32_t col = j + c;
+      if (WHOLE || col < v ? (int32_t)col == t : (int32_t)(col - v) == u) g[c] = g[c] - 1.0f;
+      g[c] = g[c] * scale;
+    }
+    __builtin_nontemporal_store(g, reinterpret_cast<v4f*>(dx) + f4);
+  }
+  if (!WHOLE && id < total - 4 * total4) {  // in the last row
+    const uint32_t f = 4 * total4 + id, j = f - (n - 1) * v;
+    float g = probs[f];
+    if ((int32_t)j == tgt[n - 1]) g = g - 1.0f;
+    dx[f] = g * scale;
   }
 }
 
@@ -612,38 +661,65 @@ __global__ void k_ce_fwd_seq(const float* __restrict__ logits, const int32_t* __
 // step's <= 100 MB operands cached loads are faster).
 constexpr size_t kStreamBytes = 256ull << 20;
 
-template <template <int, int> class KSel, class Launch>
-void row_dispatch(uint32_t axis, Launch launch, size_t bytes = 0) {
-  const bool vec = (axis % 4) == 0;
+// One wave per row up to kWaveRowAxis: beyond, its 128 values a lane (two
+// tiles of 64) leave few waves in flight, and a workgroup per row with 16
+// values a thread is faster (layernorm forward + backward 16384 x 4096 201 ->
+// 195 us, 20000 x 3333 256 -> 234, 2000 x 4096 29.4 -> 26.8; cross-entropy 20000 x
+// 3333 202 -> 170), while at 40000 x 1500 it is 1 % slower.  Rows past 4096
+// took the sequential kernel's one thread per row before (8192 x 8192: layernorm
+// 12930 -> 197 us, cross-entropy 6860 -> 169; 8000 x 5003: 18730 -> 144 and 8950 ->
+// 116), which still runs past kMaxRowAxis, where 1024 threads hold no whole
+// row in 16 registers each.  aligned: every operand is at 16 bytes (the
+// workgroup forms load 16 bytes only then).
+constexpr uint32_t kWaveRowAxis = 2048, kMaxRowAxis = 16384;
+
+template <template <int, int, int> class KSel, class Launch>
+void row_dispatch(uint32_t axis, Launch launch, size_t bytes, bool aligned) {
+  const bool vec = axis % 4 == 0 && (axis <= kWaveRowAxis || aligned);
   const bool nt = bytes >= kStreamBytes;
   // elements per lane needed: ceil(axis / 64)
   uint32_t per_lane = (axis + 63) / 64;
-  int nv = per_lane <= 4 ? 1 : per_lane <= 8 ? 2 : per_lane <= 16 ? 4 : per_lane <= 32 ? 8 : 16;
-#define MALUS_ROW_CASE(NV)                                       \
-  case NV:                                                       \
-    if (vec && nt) launch(KSel<NV, 2>{});                             \
-    else if (vec) launch(KSel<NV, 1>{});                             \
-    else launch(KSel<NV, 0>{});                                      \
-    break;
+  int nv = per_lane <= 4 ? 1 : per_lane <= 8 ? 2 : per_lane <= 16 ? 4 : 8;
+#define MALUS_ROW_CASE(NV, W)                                    \
+  {                                                              \
+    if (vec && nt) launch(KSel<NV, 2, W>{});                     \
+    else if (vec) launch(KSel<NV, 1, W>{});                      \
+    else launch(KSel<NV, 0, W>{});                               \
+    return;                                                      \
+  }
+  if (axis > kWaveRowAxis) {
+    if (axis <= 4096) MALUS_ROW_CASE(4, 256)
+    if (axis <= 8192) MALUS_ROW_CASE(4, 512)
+    MALUS_ROW_CASE(4, 1024)
+  }
   switch (nv) {
-    MALUS_ROW_CASE(1)
-    MALUS_ROW_CASE(2)
-    MALUS_ROW_CASE(4)
-    MALUS_ROW_CASE(8)
-    MALUS_ROW_CASE(16)
+    case 1: MALUS_ROW_CASE(1, kWave)
+    case 2: MALUS_ROW_CASE(2, kWave)
+    case 4: MALUS_ROW_CASE(4, kWave)
+    default: MALUS_ROW_CASE(8, kWave)
   }
 #undef MALUS_ROW_CASE
 }
 
-template <int NV, int VM> struct SelSoftmax { static constexpr auto fn = k_softmax_rows<NV, VM>; };
-template <int NV, int VM> struct SelSoftmaxBwd { static constexpr auto fn = k_softmax_bwd_rows<NV, VM>; };
-template <int NV, int VM> struct SelScaleMaskSoftmax { static constexpr auto fn = k_scale_mask_softmax_rows<NV, VM>; };
-template <int NV, int VM> struct SelLN { static constexpr auto fn = k_layernorm_rows<NV, VM>; };
-template <int NV, int VM> struct SelLNBwd { static constexpr auto fn = k_layernorm_bwd_rows<NV, VM>; };
-template <int NV, int VM> struct SelCE { static constexpr auto fn = k_ce_fwd_rows<NV, VM>; };
+template <int W>
+struct RowLaunch {
+  static constexpr unsigned threads = W == kWave ? 256 : W;
+  static unsigned grid(size_t rows) { return (unsigned)(W == kWave ? (rows + kRowsPerBlock - 1) / kRowsPerBlock : rows); }
+};
+template <int NV, int VM, int W> struct SelSoftmax : RowLaunch<W> { static constexpr auto fn = k_softmax_rows<NV, VM, W>; };
+template <int NV, int VM, int W> struct SelSoftmaxBwd : RowLaunch<W> { static constexpr auto fn = k_softmax_bwd_rows<NV, VM, W>; };
+template <int NV, int VM, int W> struct SelLN : RowLaunch<W> { static constexpr auto fn = k_layernorm_rows<NV, VM, W>; };
+template <int NV, int VM, int W> struct SelLNBwd : RowLaunch<W> { static constexpr auto fn = k_layernorm_bwd_rows<NV, VM, W>; };
+template <int NV, int VM, int W> struct SelCE : RowLaunch<W> { static constexpr auto fn = k_ce_fwd_rows<NV, VM, W>; };
 
-constexpr uint32_t kMaxRowAxis = 4096;
-inline unsigned row_grid(size_t rows) { return (unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock); }
+template <int NV, int VM, int W> struct SelScaleMaskSoftmax : RowLaunch<W> {
+  static constexpr auto fn = k_scale_mask_softmax_rows<NV, VM, W>;
+};
+
+template <class... P>
+bool aligned16(const P*... p) {
+  return ((reinterpret_cast<uintptr_t>(p) | ...) & 15) == 0;
+}
 inline unsigned seq_grid(size_t n) { return (unsigned)((n + 255) / 256); }
 
 }  // namespace
@@ -652,8 +728,8 @@ void softmax(const float* x, float* out, size_t outer, size_t axis, size_t inner
   if (!outer || !axis || !inner) return;
   if (inner == 1 && axis <= kMaxRowAxis) {
     row_dispatch<SelSoftmax>((uint32_t)axis, [&](auto sel) {
-      decltype(sel)::fn<<<row_grid(outer), 256, 0, s>>>(x, out, outer, (uint32_t)axis);
-    }, 2 * outer * (size_t)axis * sizeof(float));
+      decltype(sel)::fn<<<sel.grid(outer), sel.threads, 0, s>>>(x, out, outer, (uint32_t)axis);
+    }, 2 * outer * (size_t)axis * sizeof(float), aligned16(x, out));
   } else {
     k_softmax_seq<<<seq_grid(outer * inner), 256, 0, s>>>(x, out, outer, axis, inner);
   }
@@ -665,8 +741,8 @@ void scale_mask_softmax(const float* S, const float* scale, const float* mask, f
   if (!rows || !axis) return;
   if (axis <= kMaxRowAxis && mask_rows > 0) {
     row_dispatch<SelScaleMaskSoftmax>((uint32_t)axis, [&](auto sel) {
-      decltype(sel)::fn<<<row_grid(rows), 256, 0, s>>>(S, scale, mask, P, rows, (uint32_t)axis, (uint32_t)mask_rows);
-    }, 2 * rows * (size_t)axis * sizeof(float));
+      decltype(sel)::fn<<<sel.grid(rows), sel.threads, 0, s>>>(S, scale, mask, P, rows, (uint32_t)axis, (uint32_t)mask_rows);
+    }, 2 * rows * (size_t)axis * sizeof(float), aligned16(S, mask, P));
     MALUS_HIP(hipGetLastError());
     return;
   }
@@ -684,8 +760,8 @@ void softmax_bwd(const float* y, const float* dout, float* out, size_t outer, si
   if (!outer || !axis || !inner) return;
   if (inner == 1 && axis <= kMaxRowAxis) {
     row_dispatch<SelSoftmaxBwd>((uint32_t)axis, [&](auto sel) {
-      decltype(sel)::fn<<<row_grid(outer), 256, 0, s>>>(y, dout, out, outer, (uint32_t)axis);
-    }, 3 * outer * (size_t)axis * sizeof(float));
+      decltype(sel)::fn<<<sel.grid(outer), sel.threads, 0, s>>>(y, dout, out, outer, (uint32_t)axis);
+    }, 3 * outer * (size_t)axis * sizeof(float), aligned16(y, dout, out));
   } else {
     k_softmax_bwd_seq<<<seq_grid(outer * inner), 256, 0, s>>>(y, dout, out, outer, axis, inner);
   }
@@ -716,8 +792,8 @@ void layernorm(const float* x, float* y, float* var, size_t outer, size_t axis, 
     }
   } else if (inner == 1 && axis <= kMaxRowAxis) {
     row_dispatch<SelLN>((uint32_t)axis, [&](auto sel) {
-      decltype(sel)::fn<<<row_grid(outer), 256, 0, s>>>(x, y, var, outer, (uint32_t)axis, eps, w, out);
-    }, (w ? 3 : 2) * outer * (size_t)axis * sizeof(float));
+      decltype(sel)::fn<<<sel.grid(outer), sel.threads, 0, s>>>(x, y, var, outer, (uint32_t)axis, eps, w, out);
+    }, (w ? 3 : 2) * outer * (size_t)axis * sizeof(float), aligned16(x, y, w, out));
   } else {
     if (w) fail("malus: fused layernorm scale needs the normalized axis last");
     k_layernorm_seq<<<seq_grid(outer * inner), 256, 0, s>>>(x, y, var, outer, axis, inner, eps);
@@ -739,8 +815,8 @@ void layernorm_bwd(const float* y, const float* var, const float* dout, float* d
     }
   } else if (inner == 1 && axis <= kMaxRowAxis) {
     row_dispatch<SelLNBwd>((uint32_t)axis, [&](auto sel) {
-      decltype(sel)::fn<<<row_grid(outer), 256, 0, s>>>(y, var, dout, dx, outer, (uint32_t)axis, eps, addend, w);
-    }, 3 * outer * (size_t)axis * sizeof(float));
+      decltype(sel)::fn<<<sel.grid(outer), sel.threads, 0, s>>>(y, var, dout, dx, outer, (uint32_t)axis, eps, addend, w);
+    }, 3 * outer * (size_t)axis * sizeof(float), aligned16(y, dout, dx, addend, w));
   } else {
     if (w) fail("malus: fused layernorm scale needs the normalized axis last");
     k_layernorm_bwd_seq<<<seq_grid(outer * inner), 256, 0, s>>>(y, var, dout, dx, outer, axis, inner, eps);
@@ -777,8 +853,8 @@ void ce_fwd(const float* logits, const int32_t* tgt, float* probs, float* nll, s
   if (!n || !v) return;
   if (v <= kMaxRowAxis) {
     row_dispatch<SelCE>((uint32_t)v, [&](auto sel) {
-      decltype(sel)::fn<<<row_grid(n), 256, 0, s>>>(logits, tgt, probs, nll, n, (uint32_t)v, err);
-    }, 2 * n * (size_t)v * sizeof(float));
+      decltype(sel)::fn<<<sel.grid(n), sel.threads, 0, s>>>(logits, tgt, probs, nll, n, (uint32_t)v, err);
+    }, 2 * n * (size_t)v * sizeof(float), aligned16(logits, probs));
   } else {
     k_ce_fwd_seq<<<seq_grid(n), 256, 0, s>>>(logits, tgt, probs, nll, n, v, err);
   }
@@ -789,11 +865,11 @@ void ce_bwd(const float* probs, const int32_t* tgt, const float* dout, float sca
             hipStream_t s) {
   size_t total = n * v;
   if (!total) return;
-  if (v % 4 == 0 && total < (1ull << 32)) {
-    const size_t total4 = total / 4;
-    size_t blocks = (total4 + 255) / 256;
+  if (v >= 4 && total < (1ull << 32) && aligned16(probs, dx)) {
+    size_t blocks = (total / 4 + 255) / 256;
     if (blocks > (1u << 20)) blocks = 1u << 20;
-    k_ce_bwd4<<<(unsigned)blocks, 256, 0, s>>>(probs, tgt, dout, scale_host, dx, (uint32_t)n, (uint32_t)v, (uint32_t)total4);
+    const auto fn = v % 4 == 0 ? k_ce_bwd4<true> : k_ce_bwd4<false>;
+    fn<<<(unsigned)blocks, 256, 0, s>>>(probs, tgt, dout, scale_host, dx, (uint32_t)n, (uint32_t)v, (uint32_t)total);
     MALUS_HIP(hipGetLastError());
     return;
   }

@@ -477,6 +477,60 @@ def test_cross_entropy_fwd_bwd(rt, n, v):
     rt.free(hl, ht, hloss, hp.value, hd)
 
 
+# Rows past a wave's 2048 columns run a workgroup per row up to 16384, one
+# thread per row beyond; odd widths take 4-byte accesses.  Against float64: a
+# value passes 16 + 6 + 16 roundings of a workgroup's sums and about 10 more
+# (2^-24 each: 3e-6); a thread's sequence of n passes n, all of one direction
+# where half of the row is one value: n 2^-24.
+@pytest.mark.parametrize("rows", [1, 5])
+@pytest.mark.parametrize("cols", [2047, 2048, 2049, 2052, 4095, 4096, 4097, 4100, 8191, 8192, 8193, 8196, 16383, 16384, 16385])
+def test_wide_rows(rt, rows, cols):
+    tol = 3e-6 if cols <= 16384 else cols * 2.0 ** -24
+    x = rand(rows, cols, lo=-3, hi=3) + 0.5
+    x[0, cols // 2:] = -1e9  # a masked tail
+    d = rand(rows, cols)
+    t = RNG.integers(0, cols, rows).astype(np.int32)
+    t[0], t[-1] = 0, min(t[-1], cols // 2 - 1)
+    hx, hd, ht, one = rt.tensor(x), rt.tensor(d), rt.tensor(t), rt.tensor(np.array([1.0], np.float32))
+    e = np.exp(x.astype(np.float64) - x.max(1, keepdims=True))
+    p64 = e / e.sum(1, keepdims=True)
+    hy = rt.L.malus_std_softmax_fwd(hx, 1)
+    y = rt.numpy(hy)
+    assert_normwise(y, p64, tol, "softmax")
+    y64 = y.astype(np.float64)
+    got = run(rt, rt.L.malus_std_softmax_bwd(hy, hd, 1))
+    assert_normwise(got, y64 * (d - (d * y64).sum(1, keepdims=True)), tol, "softmax bwd")
+    hp = C.c_int64()
+    hloss = rt.L.malus_std_cross_entropy_fwd(hx, ht, C.byref(hp))
+    loss, probs = rt.numpy(hloss), rt.numpy(hp.value)
+    assert np.array_equal(probs, y)
+    assert_normwise(loss, [-np.log(p64[np.arange(rows), t]).mean()], tol, "loss")
+    got = run(rt, rt.L.malus_std_cross_entropy_bwd(hp.value, ht, one))
+    assert_normwise(got, O.cross_entropy_bwd(probs, t, 1.0), 1e-6, "ce bwd")
+    x[0, cols // 2:] = 0.25
+    hz, hv = rt.tensor(x), C.c_int64()
+    hn = rt.L.malus_std_layernorm_fwd(hz, 1, C.byref(hv))
+    n, var = rt.numpy(hn), rt.numpy(hv.value)
+    x64 = x.astype(np.float64)
+    v64 = x64.var(1)
+    assert_normwise(var.ravel(), v64, tol, "layernorm var")
+    assert_normwise(n, (x64 - x64.mean(1, keepdims=True)) / np.sqrt(v64 + 1e-5)[:, None], tol, "layernorm y")
+    n64 = n.astype(np.float64)
+    want = (d - d.mean(1, keepdims=True, dtype=np.float64) - n64 * (d * n64).mean(1, keepdims=True))
+    got = run(rt, rt.L.malus_std_layernorm_bwd(hn, hv.value, hd, 1))
+    assert_normwise(got, want / np.sqrt(var.astype(np.float64).reshape(rows, 1) + 1e-5), tol, "layernorm bwd")
+    rt.free(hx, hd, ht, one, hy, hloss, hp.value, hz, hn, hv.value)
+
+
+@pytest.mark.parametrize("n,v", [(1, 4), (3, 5), (7, 6), (50, 65), (1, 3), (9, 2), (5, 1), (33, 1021), (6, 4099)])
+def test_cross_entropy_bwd_ragged(rt, n, v):
+    probs, t = rand(n, v, lo=0, hi=1), RNG.integers(0, v, n).astype(np.int32)
+    hp, ht, hd = rt.tensor(probs), rt.tensor(t), rt.tensor(np.array([0.7], np.float32))
+    got = run(rt, rt.L.malus_std_cross_entropy_bwd(hp, ht, hd))
+    assert_normwise(got, O.cross_entropy_bwd(probs, t, np.float32(0.7)), 1e-6, "ce bwd")
+    rt.free(hp, ht, hd)
+
+
 # ------------------------------------------------------------ index ops
 @pytest.mark.parametrize("v,d,t", [(65, 384, 4096), (256, 384, 2048), (65, 65, 777), (4, 3, 4), (3, 128, 16384),
                                    (65, 384, 4097), (2048, 64, 9000), (400, 32, 4096), (65, 384, 16384), (256, 384, 16384),

@@ -182,6 +182,22 @@ def test_gpt_fusions_equal_separate_ops(rt, cfg):
         np.testing.assert_array_equal(pa[i], pb[i], err_msg=f"param {i}")
 
 
+@pytest.mark.parametrize("t", [2049, 2052, 4112])
+def test_fused_scores_on_wide_rows(rt, t):
+    """Scale + mask + softmax in one kernel with a workgroup per row equals the
+    separate ops, bit for bit (head size 16 takes the composed scores)."""
+    cfg = dict(V=16, T=t, C=16, H=1, L=1, B=1)
+    x, y = tokens(cfg, 6500)
+    losses = []
+    for fused in (True, False):
+        g = GpuGpt(rt, cfg, fused_forward=fused)
+        try:
+            losses.append(g.loss_and_grads(x, y))
+        finally:
+            g.close()
+    assert losses[0] == losses[1] and np.isfinite(losses[0])
+
+
 @pytest.mark.parametrize("cfg", [dict(V=65, T=256, C=128, H=2, L=2, B=2),
                                  dict(V=65, T=128, C=256, H=4, L=1, B=3)], ids=["t256hs64", "t128hs64"])
 def test_fused_attention_unwritten_tiles(rt, cfg):
