@@ -602,6 +602,17 @@ def test_transpose_2d(rt, shape):
     rt.free(hx)
 
 
+# one element per thread up to 65536 elements, 64 x 64 tiles beyond
+@pytest.mark.parametrize("shape", [(1, 5), (4, 8), (3, 65, 7), (256, 256), (257, 255), (1, 65537), (5, 63, 209)])
+def test_transpose_element_edge(rt, shape):
+    x = rand(*shape)
+    hx = rt.tensor(x)
+    perm = list(range(len(shape) - 2)) + [len(shape) - 1, len(shape) - 2]
+    got = run(rt, rt.L.tensor_permute(hx, M.sizes(perm), len(shape)))
+    assert_bitexact(got, x.transpose(perm), f"transpose {shape}")
+    rt.free(hx)
+
+
 def test_permute_3d_batched_transpose(rt):
     x = rand(384, 64, 256)
     hx = rt.tensor(x)
