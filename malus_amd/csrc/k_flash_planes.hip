@@ -12,8 +12,7 @@
 // during the current tile's products and one barrier per tile.  Both
 // orientations are read from the same planes: rows with 128-bit reads,
 // columns with gfx950's transposing read (ds_read_b64_tr_b16).
-// The products run in the order of the per-wave form, so the values are the
-// same bit for bit.
+// The products run in the order of the per-wave form; only exp differs.
 #include "k_flash.h"
 
 namespace malus {
