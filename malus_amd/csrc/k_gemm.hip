@@ -518,7 +518,8 @@ double best_x3_tile(int M, int N, int K, bool split_ok, int groups, Plan* best) 
 
 // The plan of a split product; ti < 0: the kernels of k_gemm_dma.h, which
 // keep the batched products (the composed attention's, K = T or the head
-// size), K < 128 (the slabs in flight are then most of the K loop: 2048 x 512 x
+// size; a batch of one too, so that one head has the bits of many, and of the
+// fused attention kernels), K < 128 (the slabs in flight are then most of the K loop: 2048 x 512 x
 // 128 takes 7.7 us here and 7.2 there) and the tuning knobs' tiles and
 // splits.  groups: the products one grouped launch runs side by side.  They
 // do not change a split, so that a grouped product has the bits of the
@@ -528,10 +529,10 @@ double best_x3_tile(int M, int N, int K, bool split_ok, int groups, Plan* best) 
 // 8.5, 128 x 4096 x 1024 18.8 -> 12.4) and lose to a split K from 96 slabs on (256
 // x 384 x 1536 13.0 against 14.4) and in a second round (2048 x 384 x 384,
 // B transposed, 11.8 against 19.6).
-Plan plan_x3(int batch, int M, int N, int K, bool split_ok, int groups) {
+Plan plan_x3(bool batched, int M, int N, int K, bool split_ok, int groups) {
   Plan best{-1, 1, K};
   read_forced_tile();
-  if (g_forced_tile >= 0 || g_split_target > 0 || batch > 1 || K < 128) return best;
+  if (g_forced_tile >= 0 || g_split_target > 0 || batched || K < 128) return best;
   if ((long)((M + 31) / 32) * ((N + 63) / 64) <= 256) {
     const double waves = (K / BK + 7) / 8 * 0.78 + 3.8;
     if (waves < best_x3_tile(M, N, K, true, 1, &best)) return Plan{kX3K, 1, K};
@@ -626,7 +627,10 @@ double launch_dma(const float* A, const float* B, float* C, int batch, int M, in
   if ((L.io & kIoC16) && D) fail("malus: gemm: a bf16 output takes no addend");
   if (epi || (L.io & kIoC16)) split_ok = false;
   Plan p{-1, 1, K};
-  if (x3 && !(mapped && L.tri_a)) p = plan_x3(batch, M, N, K, split_ok, 1);
+  // a product of batches has a batch stride, whatever the number of batches
+  const auto strided = [](const GemmMap& b) { return b.s0 != 0 || b.s1 != 0; };
+  const bool batched = batch > 1 || strided(L.a.b) || strided(L.b.b);
+  if (x3 && !(mapped && L.tri_a)) p = plan_x3(batched, M, N, K, split_ok, 1);
   const bool once = p.ti >= 0;  // each value split once per workgroup
   if (!once) {
     // Under autocast the GELU GEMM (h = x W1, K = 384, a 3072-workgroup grid
@@ -759,7 +763,7 @@ bool gemm_grouped(int M, int N, int K, bool transA, bool transB, const GemmLayou
   const bool c_dense = L.c.r.div == 0 && L.c.c.div == 0 && L.c.c.s0 == 1 && L.c.r.s0 == N;
   const bool split_ok = !accumulate && c_dense && !(L.io & kIoC16);  // split partials are f32 and dense
   Plan p{-1, 1, K};
-  if (x3) p = plan_x3(1, M, N, K, split_ok, accumulate ? 1 : L.ngroup);
+  if (x3) p = plan_x3(false, M, N, K, split_ok, accumulate ? 1 : L.ngroup);
   const bool once = p.ti >= 0;  // each value split once per workgroup
   if (!once) {
     p = plan_gemm(1, M, N, K, v, false, -1, bf);

@@ -276,14 +276,15 @@ def test_attn_scores_bwd_equals_composed_ops(rt, t, hs, causal):
     rt.free(hq, hk, hv, hd, hsc, hm, hp, hvt, hdp, hdx)
 
 
-@pytest.mark.parametrize("t,hs,causal", [(256, 64, 1), (256, 64, 0), (128, 64, 1), (64, 32, 1), (64, 32, 0),
-                                          (64, 64, 0)])
-def test_attn_fwd_equals_composed_ops(rt, t, hs, causal):
+@pytest.mark.parametrize("t,hs,causal,bh", [(256, 64, 1, 6), (256, 64, 0, 6), (128, 64, 1, 6), (64, 32, 1, 6),
+                                             (64, 32, 0, 6), (64, 64, 0, 6), (256, 64, 1, 1), (256, 64, 0, 1),
+                                             (128, 64, 1, 1)])
+def test_attn_fwd_equals_composed_ops(rt, t, hs, causal, bh):
     # nanogpt_modular.ml:57-62: attn @ V with attn the fused scores softmax.
     # P @ V runs from the scores kernel's registers; it equals the batched
     # matmul of the stored P with V bit for bit (a causal P's zeros above the
-    # diagonal add exact zeros in the matmul)
-    bh = 6
+    # diagonal add exact zeros in the matmul).  One head: a batch of one
+    # product sums in the order of a batch of many.
     q, kk, v = (rand(bh, t, hs, lo=-2, hi=2) for _ in range(3))
     mask = O.causal_mask(t) if causal else rand(t, t, lo=-3, hi=3)
     sc = np.array([[1.0 / np.sqrt(hs)]], np.float32)
@@ -323,7 +324,8 @@ def test_attn_bwd_dq_equals_composed_ops(rt, t, hs, causal):
 
 
 @pytest.mark.parametrize("t,hs,causal,bh", [(256, 64, 1, 5), (256, 64, 0, 5), (128, 64, 1, 5), (64, 32, 1, 5),
-                                             (64, 64, 0, 5), (256, 64, 1, 300), (64, 32, 0, 600)])
+                                             (64, 64, 0, 5), (256, 64, 1, 300), (64, 32, 0, 600),
+                                             (256, 64, 1, 1), (256, 64, 0, 1), (128, 64, 1, 1)])
 def test_attn_bwd_all_equals_composed_ops(rt, t, hs, causal, bh):
     # The whole attention VJP from one kernel: dS and dQ as the kernel
     # without the key-side products; dK and dV as the composed ops of
