@@ -140,7 +140,7 @@ def test_fused_attention_equals_composed_ops_on_fp32_mfma(rt, t, hs, causal):
     from tests import test_kernels_gpu as K
 
     with split_mode(rt, False):
-        K.test_attn_fwd_equals_composed_ops(rt, t, hs, causal)
+        K.test_attn_fwd_equals_composed_ops(rt, t, hs, causal, 6)
         K.test_attn_bwd_all_equals_composed_ops(rt, t, hs, causal, 5)
 
 
@@ -162,32 +162,36 @@ def test_set_f32_split_returns_previous(rt):
         L.malus_gemm_set_f32_split(prev)
 
 
-def test_weight_split_copies_give_the_same_steps(rt):
-    # With split products the model's forward GEMMs read B from split copies
-    # of the block weights (three bf16 planes, refreshed each forward)
-    # instead of splitting the weights themselves: three steps
-    # with the copies (malus_gpt_set_bf16_activations 1, the default) equal
-    # three without, bit for bit (losses, parameters and both moments).
-    from tests.test_models_gpu import GpuGpt, tokens
-
-    cfg = dict(V=65, T=64, C=128, H=4, L=2, B=8)
-    x, y = tokens(cfg, 777)
-    out = []
+@pytest.mark.parametrize("form", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("m,n,k", [(2100, 1540, 160), (4100, 3080, 176), (16384, 384, 400), (2048, 1024, 512),
+                                   (1060, 1028, 992)])
+def test_split_once_equals_the_split_of_every_wave(rt, form, m, n, k):
+    # Splitting a value once per workgroup changes no piece and no sum: without
+    # a K split (K < 1024) and past the few tiles whose waves share K, the
+    # products have the bits of the kernels whose waves split what they read,
+    # which a pinned tile selects.
+    a = RNG.uniform(-1, 1, (m, k)).astype(np.float32)
+    b = RNG.uniform(-1, 1, (k, n)).astype(np.float32)
+    ha = rt.tensor(a if form != "tn" else np.ascontiguousarray(a.T))
+    hb = rt.tensor(b if form != "nt" else np.ascontiguousarray(b.T))
+    like = rt.tensor(np.zeros((m, n), np.float32))
+    L, got = rt.L, []
     with split_mode(rt, True):
-        for copies in (1, 0):
-            g = GpuGpt(rt, cfg)
-            try:
-                rt.L.malus_gpt_set_bf16_activations(g.g, copies)
-                losses = [g.step(x, y, t) for t in (1, 2, 3)]
-                state = [g.param(i) for i in range(8 * cfg["L"] + 4)]
-                state += [rt.numpy(rt.L.malus_gpt_moment(g.g, i, m)).ravel() for m in (0, 1)
-                          for i in range(8 * cfg["L"] + 4)]
-            finally:
-                g.close()
-            out.append((losses, state))
-    assert out[0][0] == out[1][0]
-    for i, (u, v) in enumerate(zip(out[0][1], out[1][1])):
-        np.testing.assert_array_equal(u, v, err_msg=f"state {i}")
+        try:
+            for tile in ((0, 0), (2, 1)):
+                assert L.malus_gemm_set_tile(*tile)
+                if form == "nn":
+                    out = L.tensor_matmul(ha, hb)
+                elif form == "nt":
+                    out = L.malus_std_matmul_bwd_a(like, hb, ha)
+                else:
+                    out = L.malus_std_matmul_bwd_b(ha, like, hb)
+                got.append(rt.numpy(out))
+                rt.free(out)
+        finally:
+            L.malus_gemm_set_tile(0, 0)
+    rt.free(ha, hb, like)
+    assert_bitexact(got[0], got[1], f"{form} {m}x{n}x{k}")
 
 
 @pytest.mark.parametrize("form", ["nn", "nt", "tn"])
