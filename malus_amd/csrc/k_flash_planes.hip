@@ -12,7 +12,7 @@
 // during the current tile's products and one barrier per tile.  Both
 // orientations are read from the same planes: rows with 128-bit reads,
 // columns with gfx950's transposing read (ds_read_b64_tr_b16).
-// The products run in the order of the per-wave form; only exp differs.
+// The products run in the order of the per-wave form; only exp differs (exp_of).
 #include "k_flash.h"
 
 namespace malus {
@@ -48,22 +48,24 @@ __device__ __forceinline__ v16f mul(const Frag<NP>& a, const Frag<NP>& b, v16f c
   else return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[0], b.p[0], c, 0, 0, 0);
 }
 
-// exp(x).  NP = 3: 2^p for p = x log2(e) rounded, corrected by the first
-// order of what the rounding left (x - p ln 2, exact but for its last bits):
-// 6 instructions where expf, which also clamps its range, takes 13 (the
-// forward then issues 1.5k instead of 1.9k VALU cycles a block); as accurate
-// as expf.  At x = -inf the correction is NaN, which fmaxf turns into a
-// factor of the zero power.  NP = 1: without the correction, whose 2^-24 |x|
-// is far below the bf16 rounding of the product's operand.
-template <int NP>
+// exp(x): 2^p for p = x log2(e) rounded, corrected by the first order of
+// what the rounding left (x - p ln 2, exact but for its last bits): 6 or 7
+// instructions where expf, which also clamps its range, takes 13.  As accurate
+// as expf, under autocast too: the f32 row sums and the log-sum-exp are made of
+// these values, and without the correction their error grows with |x| (rms
+// 4e-7 of the value at x = -20 .. -10, 2e-6 at -80 .. -40, against 2.5e-8).
+// The correction is NaN at an infinite x; fmaxf makes a factor of the zero power
+// of it where x is never above 0 (LE0: behind the row's maximum).  Elsewhere a
+// negative correction would also make NaN of an infinite power, so where 2^p is
+// infinite or (below 2^-126) zero the factor is 1.
+template <bool LE0>
 __device__ __forceinline__ float exp_of(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const float p = x * 1.44269504f;
   const float e = __builtin_amdgcn_exp2f(p);
-  if constexpr (NP == 1) return e;
   // ln 2 = 0.693147182 - 1.90465421e-9
   const float c = __builtin_fmaf(p, 1.90465421e-9f, __builtin_fmaf(p, -0.693147182f, x));
-  return __builtin_fmaf(e, fmaxf(c, -1.0f), e);
+  return __builtin_fmaf(e, LE0 ? fmaxf(c, -1.0f) : __builtin_fabsf(p) < 128.0f ? c : 1.0f, e);
 #else
   return x;
 #endif
@@ -256,7 +258,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_fwd(const float* __r
       float ls = 0.0f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float p = exp_of<NP>(st[r] - mn);
+        const float p = exp_of<true>(st[r] - mn);
         st[r] = p;
         ls += p;
       }
@@ -363,7 +365,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dq(const float* __re
         dp = mul<NP>(Tl::row(Vs[cur], perm_row(x), kb, lk), og[kb], dp);
       }
 #pragma unroll
-      for (int r = 0; r < 16; ++r) st[r] = exp_of<NP>(st[r] * sc - L);
+      for (int r = 0; r < 16; ++r) st[r] = exp_of<false>(st[r] * sc - L);
       if (CAUSAL && j == qt) {
 #pragma unroll
         for (int r = 0; r < 16; ++r)
@@ -486,7 +488,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dkv(
       }
       // lane = key j0 + x, register r = query i0 + perm_index(r, lk)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = exp_of<NP>(s[r] * sc - Ls[cur][0][perm_index(r, lk)]);
+      for (int r = 0; r < 16; ++r) s[r] = exp_of<false>(s[r] * sc - Ls[cur][0][perm_index(r, lk)]);
       if (CAUSAL && it == kt) {
 #pragma unroll
         for (int r = 0; r < 16; ++r)

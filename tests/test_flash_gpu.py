@@ -270,3 +270,94 @@ def test_flash_ragged_wave_groups(rt, bh, t, hs, causal, path):
     for name, g, w in zip(("out", "lse", "dq", "dk", "dv"), got, want):
         err = np.linalg.norm(g - w) / np.linalg.norm(w)
         assert err <= bar, (name, err)
+
+
+@pytest.mark.parametrize("bh,t,hs,causal", [(2, 1024, 64, 0), (2, 512, 32, 1)])
+def test_flash_row_sums_do_not_depend_on_the_product_path(rt, bh, t, hs, causal):
+    # q and k with one nonzero bf16 value a row: every path's scores are the
+    # same exact f32 values, so the row sums are those of the f32 softmax
+    # under autocast too.  The split products' lse has the same bits; its rms
+    # error against float64 is within a tenth of the FP32 path's, which calls
+    # expf.
+    q, k = np.zeros((bh, t, hs), np.float32), np.zeros((bh, t, hs), np.float32)
+    q[..., 5] = RNG.integers(1, 65, (bh, t)) / 16
+    k[..., 5] = -RNG.integers(0, 129, (bh, t)) / 32
+    v = rand(bh, t, hs)
+    handles = [rt.tensor(a) for a in (q, k, v, np.array([[1.0]], np.float32))]
+    L, got = rt.L, {}
+    for path in ("split", "fp32", "autocast"):
+        split, auto = L.malus_gemm_set_f32_split(path != "fp32"), L.malus_autocast(path == "autocast")
+        try:
+            hl = C.c_int64()
+            rt.free(L.malus_std_flash_attn_fwd(*handles, causal, C.byref(hl)))
+            got[path] = run(rt, hl.value).reshape(bh, t)
+        finally:
+            L.malus_gemm_set_f32_split(split)
+            L.malus_autocast(auto)
+    rt.free(*handles)
+    s = q[..., 5].astype(np.float64)[:, :, None] * k[..., 5].astype(np.float64)[:, None, :]
+    if causal:
+        s = np.where(np.triu(np.ones((t, t), bool), 1), -np.inf, s)
+    m = s.max(2, keepdims=True)
+    want = (m + np.log(np.exp(s - m).sum(2, keepdims=True)))[..., 0]
+    rms = {p: np.sqrt(np.mean((g - want) ** 2)) for p, g in got.items()}
+    np.testing.assert_array_equal(got["autocast"], got["split"])
+    assert rms["split"] <= 1.1 * rms["fp32"], rms
+
+
+@pytest.mark.parametrize("path", ["split", "fp32", "autocast"])
+@pytest.mark.parametrize("t,hs,causal", [(96, 64, 1), (64, 32, 0), (32, 64, 1)])
+def test_flash_scores_past_the_f32_range(rt, t, hs, causal, path):
+    # Scores that overflow to -inf behind the scale leave the rows' other
+    # probabilities as they are; a NaN or an infinity in a query reaches its
+    # own row only; a log-sum-exp that makes a probability overflow gives an
+    # infinite one (split products turn an infinite operand into NaN).
+    q, k, v = np.zeros((1, t, hs), np.float32), np.zeros((1, t, hs), np.float32), rand(1, t, hs)
+    q[0, :, 0] = 1
+    k[0, :, 0] = -4
+    k[0, ::7, 0] = -1  # scores -2^126 and, times the scale, -inf
+    k[0, 0, 0] = 1
+    d = np.full((1, t, hs), 0.5, np.float32)
+    sc = np.array([[2.0 ** 126]], np.float32)
+    L = rt.L
+    split, auto = L.malus_gemm_set_f32_split(path != "fp32"), L.malus_autocast(path == "autocast")
+
+    def both(q, k, v, d, sc, lse=None):
+        hs_ = [rt.tensor(a) for a in (q, k, v, sc, d)]
+        hq, hk, hv, hsc, hd = hs_
+        hl, dq, dk, dv = (C.c_int64() for _ in range(4))
+        ho = L.malus_std_flash_attn_fwd(hq, hk, hv, hsc, causal, C.byref(hl))
+        l = hl.value if lse is None else rt.tensor(lse)
+        assert L.malus_std_flash_attn_bwd(hd, hq, hk, hv, ho, l, hsc, causal, 0, 0, 0, C.byref(dq), C.byref(dk),
+                                          C.byref(dv)) == 0
+        out = [run(rt, h) for h in (ho, hl.value, dv.value)]
+        rt.free(*hs_, dq.value, dk.value, *([l] if lse is not None else []))
+        return out
+
+    try:
+        o, lse, dv = both(q, k, v, d, sc)
+        np.testing.assert_allclose(o[0], np.broadcast_to(v[0, 0], (t, hs)), rtol=2.0 ** -8 if path == "autocast" else 1e-6)
+        np.testing.assert_array_equal(lse, np.full_like(lse, 2.0 ** 126))
+        want = np.zeros((t, hs))
+        want[0] = 0.5 * t
+        np.testing.assert_allclose(dv[0], want, rtol=1e-6)
+        one = np.array([[1.0]], np.float32)
+        clean = both(q, k, v, d, one)
+        for bad in (np.nan, np.inf, -np.inf):
+            qb = q.copy()
+            qb[0, 9, 0] = bad
+            o, lse, _ = both(qb, k, v, d, one)
+            keep = np.arange(t) != 9
+            np.testing.assert_array_equal(o[0][keep], clean[0][0][keep])
+            np.testing.assert_array_equal(lse.ravel()[keep], clean[1].ravel()[keep])
+            assert np.isnan(o[0][9]).all() and np.isnan(lse.ravel()[9])
+        low = clean[1].copy()
+        low.reshape(-1)[9] = -200.0
+        _, _, dv = both(q, k, v, d, one, low)
+        reached = np.arange(t) <= 9 if causal else np.full(t, True)
+        assert not np.isfinite(dv[0][reached]).any() and np.isfinite(dv[0][~reached]).all()
+        if path != "split":
+            assert (dv[0][reached] == np.inf).all()
+    finally:
+        L.malus_gemm_set_f32_split(split)
+        L.malus_autocast(auto)
