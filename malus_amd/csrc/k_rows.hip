@@ -31,7 +31,8 @@ __device__ __forceinline__ float wmax(float v) {
 // over it; red: one float per wave, not reused by the kernel.
 template <int W>
 __device__ __forceinline__ size_t row_index() {
-  return W == kWave ? (size_t)blockIdx.x * kRowsPerBlock + threadIdx.x / kWave : (size_t)blockIdx.x;
+  return W == kWave ? (size_t)blockIdx.x * kRowsPerBlock + threadIdx.x / kWave
+                    : (size_t)blockIdx.y * gridDim.x + blockIdx.x;
 }
 template <int W>
 __device__ __forceinline__ float rsum(float v, float* red) {
@@ -701,10 +702,17 @@ void row_dispatch(uint32_t axis, Launch launch, size_t bytes, bool aligned) {
 #undef MALUS_ROW_CASE
 }
 
+// A launch takes fewer than 2^32 threads along x: rows past that go along y
+// (2^24 rows of 2049 columns are 137 GB, so two such operands fit the card).
 template <int W>
 struct RowLaunch {
   static constexpr unsigned threads = W == kWave ? 256 : W;
-  static unsigned grid(size_t rows) { return (unsigned)(W == kWave ? (rows + kRowsPerBlock - 1) / kRowsPerBlock : rows); }
+  static constexpr dim3 grid(size_t rows) {
+    if (W == kWave) return dim3((unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock));
+    constexpr size_t max_x = 0xffffffffu / threads;
+    const size_t y = (rows + max_x - 1) / max_x;
+    return dim3((unsigned)((rows + y - 1) / y), (unsigned)y);
+  }
 };
 template <int NV, int VM, int W> struct SelSoftmax : RowLaunch<W> { static constexpr auto fn = k_softmax_rows<NV, VM, W>; };
 template <int NV, int VM, int W> struct SelSoftmaxBwd : RowLaunch<W> { static constexpr auto fn = k_softmax_bwd_rows<NV, VM, W>; };
