@@ -255,3 +255,38 @@ def test_multiply_gradients_fold_into_existing_ones(tape, shape_b):
             rt.L.malus_tape_set_fused_vjps(1)
     for f, u in zip(*got):
         assert_bitexact(f, u, "folded gradients")
+
+
+@pytest.mark.parametrize("cols", [2047, 2049, 2052, 4100, 8193, 8196, 16384, 16388])
+def test_wide_layernorm_gradient_onto_an_existing_one(tape, cols):
+    # z = layernorm(x) + x: the layernorm's VJP adds to the gradient that the
+    # sum left, in the row kernel itself (a workgroup per row past 2048
+    # columns) or, with the fused VJPs off, by an add of its own: the same
+    # bits.  (The order of the row sums is the same either way.)
+    rt = tape
+    rng = np.random.default_rng(cols)
+    x, up = (rng.standard_normal((7, cols)).astype(np.float32) for _ in range(2))
+    got = []
+    for fused in (1, 0):
+        rt.L.malus_tape_set_fused_vjps(fused)
+        try:
+            hx, hu = leaf(rt, x), leaf(rt, up)
+            hv = C.c_int64()
+            y = rt.L.malus_std_layernorm_fwd(hx, 1, C.byref(hv))
+            rt.L.tape_record_layernorm(OP["Layernorm"], hx, y, hv.value, 1)
+            z = rt.L.malus_std_broadcast_fwd(M.ADD, y, hx)
+            rt.L.tape_record_binop(OP["Add"], y, hx, z)
+            w = rt.L.malus_std_broadcast_fwd(M.MUL, z, hu)
+            rt.L.tape_record_binop(OP["Mul"], z, hu, w)
+            rt.L.backward(w)
+            got.append(grad(rt, hx))
+            rt.free(hx, hu, y, z, w)  # the tape holds the variance
+            rt.L.tape_reset()
+        finally:
+            rt.L.malus_tape_set_fused_vjps(1)
+    assert_bitexact(got[0], got[1], "layernorm gradient onto an existing one")
+    x64, u64 = x.astype(np.float64), up.astype(np.float64)
+    inv = 1 / np.sqrt(x64.var(1, keepdims=True) + 1e-5)
+    y64 = (x64 - x64.mean(1, keepdims=True)) * inv
+    want = u64 + (u64 - u64.mean(1, keepdims=True) - y64 * (u64 * y64).mean(1, keepdims=True)) * inv
+    assert_normwise(got[0], want, 3e-6 if cols <= 16384 else cols * 2.0**-24, "layernorm gradient")

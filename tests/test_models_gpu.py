@@ -198,6 +198,25 @@ def test_fused_scores_on_wide_rows(rt, t):
     assert losses[0] == losses[1] and np.isfinite(losses[0])
 
 
+@pytest.mark.parametrize("c,h", [(2049, 3), (2052, 3), (4100, 4)])
+def test_scaled_layernorm_on_wide_rows(rt, c, h):
+    """layernorm(x) * w and its VJP (onto the gradient the residual left) from
+    one kernel each, with a workgroup per row past 2048 columns, equal the
+    separate ops: the same loss and gradients, bit for bit."""
+    cfg = dict(V=16, T=16, C=c, H=h, L=1, B=2)
+    x, y = tokens(cfg, 6600)
+    got = []
+    for fused in (True, False):
+        g = GpuGpt(rt, cfg, fused_forward=fused)
+        try:
+            got.append([g.loss_and_grads(x, y)] + [g.grad(i) for i in (0, 1, 5, 8, 10)])
+        finally:
+            g.close()
+    assert np.isfinite(got[0][0])
+    for i, (a, b) in enumerate(zip(*got)):
+        np.testing.assert_array_equal(a, b, err_msg=f"output {i}")
+
+
 @pytest.mark.parametrize("cfg", [dict(V=65, T=256, C=128, H=2, L=2, B=2),
                                  dict(V=65, T=128, C=256, H=4, L=1, B=3)], ids=["t256hs64", "t128hs64"])
 def test_fused_attention_unwritten_tiles(rt, cfg):
