@@ -8,8 +8,12 @@
 // forward 3.2k VALU beside 1.5k MFMA cycles per 32 x 32 block at head size
 // 64.  Here W waves of one head, one 32-row tile each, share every streamed
 // tile: its f32 values are loaded once per workgroup, split once and kept in
-// LDS as bf16 planes, double buffered, with the next tile's loads in flight
-// during the current tile's products and one barrier per tile.  Both
+// LDS as bf16 planes.  With four waves (AHEAD) the planes are double buffered,
+// the next tile's loads are in flight during the current tile's products and a
+// tile takes one barrier.  Workgroups of one or two waves, which have a tile or
+// two to stream, keep one buffer and load between the products: the registers
+// and the LDS of the second stage cost them more waves per CU than it hides
+// (dkv at head size 64 spilled 31 registers; see dispatch for the times).  Both
 // orientations are read from the same planes: rows with 128-bit reads,
 // columns with gfx950's transposing read (ds_read_b64_tr_b16).
 // The products run in the order of the per-wave form; only exp differs (exp_of).
@@ -202,8 +206,10 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_fwd(const float* __r
                                                              const float* __restrict__ scale, float* __restrict__ O,
                                                              int ldo, int H, float* __restrict__ lse, int T, int BH) {
   constexpr int NKB = HS / 16, NN = HS / 32, NT = 64 * W;
+  constexpr bool AHEAD = W == 4 || (W == 2 && HS == 32);
+  constexpr int NB = AHEAD ? 2 : 1;
   using Tl = Tile<HS, NP>;
-  __shared__ __attribute__((aligned(1024))) char Ks[2][Tl::SIZE], Vs[2][Tl::SIZE];
+  __shared__ __attribute__((aligned(1024))) char Ks[NB][Tl::SIZE], Vs[NB][W == 1 ? 16 : Tl::SIZE];
   const int tiles = T / 32, groups = (tiles + W - 1) / W;
   const int grp = groups - 1 - (int)(blockIdx.x / BH), bh = (int)(blockIdx.x % BH);  // the longest first
   const int lane = threadIdx.x & 63, x = lane & 31, lk = lane >> 5;
@@ -214,7 +220,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_fwd(const float* __r
   const float *Kh = at<S16>(K, head), *Vh = at<S16>(V, head);
   const int i0 = 32 * qt;
   const float sc = scale[0];
-  const int jmax = CAUSAL ? min(W * grp + W, tiles) - 1 : tiles - 1;
+  const int jmax = W == 1 ? 0 : CAUSAL ? min(W * grp + W, tiles) - 1 : tiles - 1;  // W = 1: the only tile
   const int last = !live ? -1 : CAUSAL ? qt : tiles - 1;
 
   Stream<HS, NT, S16> kst, vst;
@@ -229,11 +235,11 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_fwd(const float* __r
   for (int n = 0; n < NN; ++n) o[n] = v16f{0};
   float m = -INFINITY, l = 0.0f;
   kst.template store<NP>(Ks[0]);
-  vst.template store<NP>(Vs[0]);
+  if (W > 1) vst.template store<NP>(Vs[0]);
   __syncthreads();
   for (int j = 0; j <= jmax; ++j) {
-    const int cur = j & 1;
-    if (j < jmax) {
+    const int cur = AHEAD ? j & 1 : 0;
+    if (AHEAD && j < jmax) {
       kst.fetch(Kh, HS, j + 1);
       vst.fetch(Vh, HS, j + 1);
     }
@@ -267,6 +273,13 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_fwd(const float* __r
       m = mn;
 #pragma unroll
       for (int n = 0; n < NN; ++n) o[n] *= alpha;
+      const char* vs = Vs[cur];
+      if constexpr (W == 1) {  // V takes K's place: half the LDS, twice the waves
+        __syncthreads();
+        vst.template store<NP>(Ks[0]);
+        __syncthreads();
+        vs = Ks[0];
+      }
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         float pb[8];
@@ -274,12 +287,17 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_fwd(const float* __r
         for (int e = 0; e < 8; ++e) pb[e] = st[8 * h + e];
         const Frag<NP> p = make_frag<NP>(pb);
 #pragma unroll
-        for (int n = 0; n < NN; ++n) o[n] = mul<NP>(Tl::col(Vs[cur], n, h), p, o[n]);
+        for (int n = 0; n < NN; ++n) o[n] = mul<NP>(Tl::col(vs, n, h), p, o[n]);
       }
     }
-    if (j < jmax) {
-      kst.template store<NP>(Ks[cur ^ 1]);
-      vst.template store<NP>(Vs[cur ^ 1]);
+    if (W > 1 && j < jmax) {
+      if (!AHEAD) {
+        kst.fetch(Kh, HS, j + 1);
+        vst.fetch(Vh, HS, j + 1);
+        __syncthreads();  // tile j is read
+      }
+      kst.template store<NP>(Ks[AHEAD ? cur ^ 1 : 0]);
+      vst.template store<NP>(Vs[AHEAD ? cur ^ 1 : 0]);
     }
     __syncthreads();  // tile j is read, tile j + 1 is staged
   }
@@ -309,8 +327,10 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dq(const float* __re
                                                             const float* __restrict__ Dq, float* __restrict__ dsum,
                                                             int T, int BH) {
   constexpr int NKB = HS / 16, NN = HS / 32, NT = 64 * W;
+  constexpr bool AHEAD = W == 4;
+  constexpr int NB = AHEAD ? 2 : 1;
   using Tl = Tile<HS, NP>;
-  __shared__ __attribute__((aligned(1024))) char Ks[2][Tl::SIZE], Vs[2][Tl::SIZE];
+  __shared__ __attribute__((aligned(1024))) char Ks[NB][Tl::SIZE], Vs[NB][Tl::SIZE];
   const int tiles = T / 32, groups = (tiles + W - 1) / W;
   const int grp = groups - 1 - (int)(blockIdx.x / BH), bh = (int)(blockIdx.x % BH);
   const int lane = threadIdx.x & 63, x = lane & 31, lk = lane >> 5;
@@ -321,7 +341,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dq(const float* __re
   const float *Kh = at<S16>(K, head), *Vh = at<S16>(V, head);
   const int i0 = 32 * qt, i = live ? i0 + x : 0;
   const float sc = scale[0];
-  const int jmax = CAUSAL ? min(W * grp + W, tiles) - 1 : tiles - 1;
+  const int jmax = W == 1 ? 0 : CAUSAL ? min(W * grp + W, tiles) - 1 : tiles - 1;
   const int last = !live ? -1 : CAUSAL ? qt : tiles - 1;
 
   Stream<HS, NT, S16> kst, vst;
@@ -352,8 +372,8 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dq(const float* __re
   vst.template store<NP>(Vs[0]);
   __syncthreads();
   for (int j = 0; j <= jmax; ++j) {
-    const int cur = j & 1;
-    if (j < jmax) {
+    const int cur = AHEAD ? j & 1 : 0;
+    if (AHEAD && j < jmax) {
       kst.fetch(Kh, HS, j + 1);
       vst.fetch(Vh, HS, j + 1);
     }
@@ -387,9 +407,14 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dq(const float* __re
         for (int n = 0; n < NN; ++n) dq[n] = mul<NP>(ds, Tl::col(Ks[cur], n, h), dq[n]);
       }
     }
-    if (j < jmax) {
-      kst.template store<NP>(Ks[cur ^ 1]);
-      vst.template store<NP>(Vs[cur ^ 1]);
+    if (W > 1 && j < jmax) {
+      if (!AHEAD) {
+        kst.fetch(Kh, HS, j + 1);
+        vst.fetch(Vh, HS, j + 1);
+        __syncthreads();  // tile j is read
+      }
+      kst.template store<NP>(Ks[AHEAD ? cur ^ 1 : 0]);
+      vst.template store<NP>(Vs[AHEAD ? cur ^ 1 : 0]);
     }
     __syncthreads();
   }
@@ -424,9 +449,11 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dkv(
     float* __restrict__ dK, const float* __restrict__ Dk, float* __restrict__ dV, const float* __restrict__ Dv, int T,
     int BH) {
   constexpr int NKB = HS / 16, NN = HS / 32, NT = 64 * W;
+  constexpr bool AHEAD = W == 4;
+  constexpr int NB = AHEAD ? 2 : 1;
   using Tl = Tile<HS, NP>;
-  __shared__ __attribute__((aligned(1024))) char Qs[2][Tl::SIZE], Os[2][Tl::SIZE];
-  __shared__ __attribute__((aligned(16))) float Ls[2][2][32];  // lse and dsum of the tile's rows
+  __shared__ __attribute__((aligned(1024))) char Qs[NB][Tl::SIZE], Os[NB][Tl::SIZE];
+  __shared__ __attribute__((aligned(16))) float Ls[NB][2][32];  // lse and dsum of the tile's rows
   const int tiles = T / 32;
   const int grp = (int)(blockIdx.x / BH), bh = (int)(blockIdx.x % BH);
   const int lane = threadIdx.x & 63, x = lane & 31, lk = lane >> 5;
@@ -472,8 +499,8 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dkv(
   store_rows(0);
   __syncthreads();
   for (int it = wg_first; it < tiles; ++it) {
-    const int cur = (it - wg_first) & 1;
-    if (it + 1 < tiles) {
+    const int cur = AHEAD ? (it - wg_first) & 1 : 0;
+    if (AHEAD && it + 1 < tiles) {
       qst.fetch(Qh, HS, it + 1);
       ost.fetch(dOh, ldo, it + 1);
       fetch_rows(it + 1);
@@ -517,10 +544,16 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dkv(
         }
       }
     }
-    if (it + 1 < tiles) {
-      qst.template store<NP>(Qs[cur ^ 1]);
-      ost.template store<NP>(Os[cur ^ 1]);
-      store_rows(cur ^ 1);
+    if (W > 1 && it + 1 < tiles) {
+      if (!AHEAD) {
+        qst.fetch(Qh, HS, it + 1);
+        ost.fetch(dOh, ldo, it + 1);
+        fetch_rows(it + 1);
+        __syncthreads();  // tile it is read
+      }
+      qst.template store<NP>(Qs[AHEAD ? cur ^ 1 : 0]);
+      ost.template store<NP>(Os[AHEAD ? cur ^ 1 : 0]);
+      store_rows(AHEAD ? cur ^ 1 : 0);
     }
     __syncthreads();
   }
@@ -570,12 +603,38 @@ void bwd_launch(const FlashBwd& a, int ldo, int H, int T, int BH, hipStream_t s)
                                                                     a.scale, a.dK, a.Dk, a.dV, a.Dv, T, BH);
 }
 
+// Waves per workgroup: one per 32-row tile up to two tiles, then four, which
+// read each streamed tile least often.  A causal group of four also waits for
+// its longest wave, and a last group of one or two tiles runs as few waves in
+// the LDS of four; with split products, where LDS and registers hold a CU to
+// two groups of four waves, two waves are then the faster group.  us at 98304 / T
+// heads, one wave a tile without shared planes / two waves / four:
+// - T = 32: forward at head size 64 20.1 / 23.5 / 28.9, one wave 18.9; backward
+//   63.5 / 64.3 / 87.2, one wave 59.5
+// - causal forward, head size 64: T = 128 31.0 / 24.8 / 29.7, 160 35.2 / 34.1 /
+//   39.5, 224 42.5 / 40.2 / 42.4, 256 42.7 / 37.6 / 35.8, 448 66.4 / 57.7 / 67.7, 512
+//   71.2 / 62.2 / 59.6; head size 32: T = 96 15.3 / 17.3 / 15.5, 128 19.3 / 16.0 /
+//   18.1, 160 21.9 / 22.1 / 23.5
+// - causal backward: T = 128 93.3 / 82.4 / 96.7, 256 133 / 111 / 123, 512 229 / 176 / 181,
+//   1024 405 / 328 / 290; head size 32: T = 256 79.2 / 63.4 / 66.2, 384 104 / 79.5 / 77.6
+// - the whole square: four at T = 96 already (backward 105 / 96.6 / 93.5)
+int group_waves(bool backward, bool causal, int planes, int hs, int T) {
+  const int tiles = T / 32, last = tiles % 4;
+  if (tiles <= 2) return tiles;
+  if (!causal || planes != 3) return 4;
+  if (backward) return T <= 8 * hs ? 2 : 4;
+  if (T >= 512) return 4;
+  return last == 1 || last == 2 || tiles == 4 || (tiles == 3 && hs == 64) ? 2 : 4;
+}
+
 // f(HS, CAUSAL, NP, S16, W) as integral constants
 template <class F>
-void dispatch(size_t hs, bool causal, int planes, bool s16, int T, F f) {
+void dispatch(bool backward, size_t hs, bool causal, int planes, bool s16, int T, F f) {
   auto waves = [&](auto HS, auto CA, auto NP, auto S) {
-    if (T > 64) f(HS, CA, NP, S, std::integral_constant<int, 4>{});
-    else f(HS, CA, NP, S, std::integral_constant<int, 2>{});
+    const int w = group_waves(backward, causal, planes, (int)hs, T);
+    if (w == 4) f(HS, CA, NP, S, std::integral_constant<int, 4>{});
+    else if (w == 2) f(HS, CA, NP, S, std::integral_constant<int, 2>{});
+    else f(HS, CA, NP, S, std::integral_constant<int, 1>{});
   };
   auto store = [&](auto HS, auto CA) {
     if (planes == 3) waves(HS, CA, std::integral_constant<int, 3>{}, std::false_type{});
@@ -594,7 +653,7 @@ void dispatch(size_t hs, bool causal, int planes, bool s16, int T, F f) {
 
 void flash_planes_fwd(size_t hs, bool causal, int planes, bool qkv_bf16, const float* Q, const float* K, const float* V,
                       const float* scale, float* O, int ldo, int H, float* lse, int T, int BH, hipStream_t s) {
-  dispatch(hs, causal, planes, qkv_bf16, T, [&](auto HS, auto CA, auto NP, auto S, auto W) {
+  dispatch(false, hs, causal, planes, qkv_bf16, T, [&](auto HS, auto CA, auto NP, auto S, auto W) {
     fwd_launch<decltype(HS)::value, decltype(CA)::value, decltype(NP)::value, decltype(S)::value, decltype(W)::value>(
         Q, K, V, scale, O, ldo, H, lse, T, BH, s);
   });
@@ -602,7 +661,7 @@ void flash_planes_fwd(size_t hs, bool causal, int planes, bool qkv_bf16, const f
 
 void flash_planes_bwd(size_t hs, bool causal, int planes, bool qkv_bf16, const FlashBwd& a, int ldo, int H, int T, int BH,
                       hipStream_t s) {
-  dispatch(hs, causal, planes, qkv_bf16, T, [&](auto HS, auto CA, auto NP, auto S, auto W) {
+  dispatch(true, hs, causal, planes, qkv_bf16, T, [&](auto HS, auto CA, auto NP, auto S, auto W) {
     bwd_launch<decltype(HS)::value, decltype(CA)::value, decltype(NP)::value, decltype(S)::value, decltype(W)::value>(
         a, ldo, H, T, BH, s);
   });

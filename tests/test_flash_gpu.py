@@ -231,10 +231,13 @@ def test_gpt_flash_steps_deterministic_and_graph_equal(rt):
 
 @pytest.mark.parametrize("path", ["split", "fp32", "autocast"])
 @pytest.mark.parametrize("causal", [1, 0], ids=["causal", "full"])
-@pytest.mark.parametrize("bh,t,hs", [(3, 32, 32), (2, 64, 64), (3, 96, 32), (2, 160, 64), (1, 416, 64), (1, 544, 32)])
+@pytest.mark.parametrize("bh,t,hs", [(3, 32, 32), (2, 64, 64), (3, 96, 32), (2, 160, 64), (1, 416, 64), (1, 544, 32),
+                                     (5, 32, 64), (3, 64, 32), (2, 96, 64), (2, 128, 32), (1, 224, 32), (1, 288, 64),
+                                     (1, 352, 32), (1, 480, 64), (1, 512, 64), (1, 576, 64)])
 def test_flash_ragged_wave_groups(rt, bh, t, hs, causal, path):
-    # Sequence lengths that end inside a workgroup's group of 32-row tiles
-    # (two or four of them), against float64.  f32: 1e-5 of the norm, as
+    # Every group of 32-row tiles (one, two or four waves) and sequence
+    # lengths that end inside one, on both sides of each length where the
+    # group changes, against float64.  f32: 1e-5 of the norm, as
     # above.  Autocast: every product rounds two operands by at most 2^-9 each
     # (rms 2^-9 / sqrt 3 together about 1.6e-3), the gradients chain three of
     # them: 1.5e-2 of the norm.
