@@ -475,17 +475,23 @@ Plan plan_gemm(int batch, int M, int N, int K, int v, bool tri = false, int only
 // ---- split products, split once per workgroup (k_gemm_x3.h) ------------------
 // The tiles with their threads, the workgroups of a CU, and the time in us
 // of one 16-deep slab: of the first workgroup of a CU (lat) and of each
-// further one there (thr).  Measured on 16384 x 384 x 1536 and its transposes
-// (128x192: 103-110 us for one workgroup of 96 slabs per CU), 8192 x 1024 x
-// 4096 (128x128: 350 us, 256x128: 320 us) and 256 x 384 x 384 (64x64: 12 us
-// for 24 slabs, one workgroup on some CUs).  The wide tiles split fewer values and
+// further one there (thr), and of a round's first loads and stores of C (start).
+// Measured on 16384 x 384 x 1536 and its transposes (128x192: 103-110 us for one
+// workgroup of 96 slabs per CU), 8192 x 1024 x 4096 (128x128: 350 us, 256x128: 320
+// us) and 256 x 384 x 384 (64x64: 12 us for 24 slabs, one workgroup on some
+// CUs); start and the 64x64 tile's thr at K < 1024 fitted to 170 products of K = 128
+// .. 1024, where the start is a third of the time: with 3 us for every tile 16384
+// x 192 x 384 (B transposed) took 128x128 tiles and 26.6 us, now 64x64 and 21.9.
+// K >= 1024 keeps thr 0.24 and 3 us a round, which chose the faster splits
+// (1536 x 384 x 16384 107 us against 118).  The wide tiles split fewer values and
 // read fewer fragments per product; which of them wins is the busiest CU's
 // share of the tiles.
-struct X3Tile { int bm, bn, threads, conc; double lat, thr; };
-constexpr X3Tile kX3Tiles[] = {{128, 192, 256, 2, 1.0, 1.0},
-                               {128, 128, 256, 2, 0.66, 0.66},
-                               {256, 128, 512, 1, 1.25, 1.25},
-                               {64, 64, 256, 4, 0.33, 0.24}};
+struct X3Tile { int bm, bn, threads, conc; double lat, thr, start; };
+constexpr X3Tile kX3Tiles[] = {{128, 192, 256, 2, 1.0, 1.0, 7.0},
+                               {128, 128, 256, 2, 0.66, 0.66, 6.2},
+                               {256, 128, 512, 1, 1.25, 1.25, 6.5},
+                               {64, 64, 256, 4, 0.33, 0.18, 4.0}};
+constexpr double kX3DeepThr64 = 0.24, kX3DeepStart = 3;
 constexpr int kX3Count = sizeof(kX3Tiles) / sizeof(kX3Tiles[0]);
 constexpr int kX3K = kX3Count;  // a plan's ti: the waves split K (k_gemm_x3k.h: 32x64 tiles of eight waves)
 
@@ -507,8 +513,8 @@ double best_x3_tile(int M, int N, int K, bool split_ok, int groups, Plan* best) 
       const int ns = (K + kc - 1) / kc;
       const long per_cu = (tiles * ns + 255) / 256;
       const long rounds = (per_cu + c.conc - 1) / c.conc;
-      // 3 us a round for the first loads and the stores of C
-      double t = (kc / BK) * (rounds * c.lat + (per_cu - rounds) * c.thr) + rounds * 3;
+      const double thr = K >= 1024 && c.bm == 64 ? kX3DeepThr64 : c.thr, start = K >= 1024 ? kX3DeepStart : c.start;
+      double t = (kc / BK) * (rounds * c.lat + (per_cu - rounds) * thr) + rounds * start;
       if (ns > 1) t += (ns + 1.0) * M * N * groups * 4.0 / 4e6 + 3;
       if (t < best_t * 0.999) { best_t = t; *best = Plan{ti, ns, kc}; }
     }
@@ -516,29 +522,43 @@ double best_x3_tile(int M, int N, int K, bool split_ok, int groups, Plan* best) 
   return best_t;
 }
 
+// The time (us) of the kernels of k_gemm_dma.h for a split product without a
+// K split: 128x64 tiles, three workgroups a CU (fitted as the tiles above).
+double x3_dma_time(int M, int N, int K, int groups) {
+  const long tiles = (long)((M + 127) / 128) * ((N + 63) / 64) * groups;
+  const long per_cu = (tiles + 255) / 256, rounds = (per_cu + 2) / 3;
+  return (K / BK) * (rounds * 0.392 + (per_cu - rounds) * 0.457) + rounds * 3.5;
+}
+
 // The plan of a split product; ti < 0: the kernels of k_gemm_dma.h, which
 // keep the batched products (the composed attention's, K = T or the head
 // size; a batch of one too, so that one head has the bits of many, and of the
-// fused attention kernels), K < 128 (the slabs in flight are then most of the K loop: 2048 x 512 x
-// 128 takes 7.7 us here and 7.2 there) and the tuning knobs' tiles and
-// splits.  groups: the products one grouped launch runs side by side.  They
-// do not change a split, so that a grouped product has the bits of the
-// single one; nor do groups, epilogues or a missing split decide for the
-// kernel whose waves split K, which needs a CU to itself: its 32 x 64 tiles
-// take 0.78 us per 8 slabs (256 x 384 x 384: 12.2 -> 7.5 us, 512^3 15.2 ->
+// fused attention kernels), the short ones (K < 128 always, K < 320 where
+// x3_dma_time says so: the slabs in flight are then most of the K loop, and 1024
+// x 2048 x 160 takes 11.5 us here and 8.9 there; the sums are the same) and the
+// tuning knobs' tiles and splits.  groups: the products one grouped launch
+// runs side by side.  They do not change a split, so that a grouped product has
+// the bits of the single one; nor do groups, epilogues or a missing split decide
+// for the kernel whose waves split K, which needs a CU to itself: its 32 x 64
+// tiles take 0.78 us per 8 slabs (256 x 384 x 384: 12.2 -> 7.5 us, 512^3 15.2 ->
 // 8.5, 128 x 4096 x 1024 18.8 -> 12.4) and lose to a split K from 96 slabs on (256
 // x 384 x 1536 13.0 against 14.4) and in a second round (2048 x 384 x 384,
-// B transposed, 11.8 against 19.6).
-Plan plan_x3(bool batched, int M, int N, int K, bool split_ok, int groups) {
+// B transposed, 11.8 against 19.6).  nt: B transposed, A not, so that a lane
+// loads 16 bytes of a row of its own: 1.3 us per 8 slabs where the rows start a
+// multiple of 128 bytes apart (K = 128: 8.2 us against 6.2 on 64x64 tiles, K = 384
+// 10.8 and 10.7, K = 640 12.9 and 15.2; K = 240, whose rows do not, 6.7 and 7.5).
+Plan plan_x3(bool batched, int M, int N, int K, bool split_ok, int groups, bool nt) {
   Plan best{-1, 1, K};
   read_forced_tile();
   if (g_forced_tile >= 0 || g_split_target > 0 || batched || K < 128) return best;
   if ((long)((M + 31) / 32) * ((N + 63) / 64) <= 256) {
-    const double waves = (K / BK + 7) / 8 * 0.78 + 3.8;
+    const int per_wave = (K / BK + 7) / 8;
+    const double waves = nt && K % 32 == 0 ? per_wave * 1.3 + 7.0 : per_wave * 0.78 + (K >= 1024 ? 3.8 : 5.2);
     if (waves < best_x3_tile(M, N, K, true, 1, &best)) return Plan{kX3K, 1, K};
   }
-  best_x3_tile(M, N, K, split_ok, split_ok ? 1 : groups, &best);
-  return best;
+  const int side_by_side = split_ok ? 1 : groups;
+  const double t = best_x3_tile(M, N, K, split_ok, side_by_side, &best);
+  return K < 320 && x3_dma_time(M, N, K, side_by_side) < t ? Plan{-1, 1, K} : best;
 }
 
 // ---- bf16 products of f32 operands, rounded once per workgroup (k_gemm_bf.h) ----
@@ -630,7 +650,7 @@ double launch_dma(const float* A, const float* B, float* C, int batch, int M, in
   // a product of batches has a batch stride, whatever the number of batches
   const auto strided = [](const GemmMap& b) { return b.s0 != 0 || b.s1 != 0; };
   const bool batched = batch > 1 || strided(L.a.b) || strided(L.b.b);
-  if (x3 && !(mapped && L.tri_a)) p = plan_x3(batched, M, N, K, split_ok, 1);
+  if (x3 && !(mapped && L.tri_a)) p = plan_x3(batched, M, N, K, split_ok, 1, !transA && transB);
   const bool once = p.ti >= 0;  // each value split once per workgroup
   if (!once) {
     // Under autocast the GELU GEMM (h = x W1, K = 384, a 3072-workgroup grid
@@ -763,7 +783,7 @@ bool gemm_grouped(int M, int N, int K, bool transA, bool transB, const GemmLayou
   const bool c_dense = L.c.r.div == 0 && L.c.c.div == 0 && L.c.c.s0 == 1 && L.c.r.s0 == N;
   const bool split_ok = !accumulate && c_dense && !(L.io & kIoC16);  // split partials are f32 and dense
   Plan p{-1, 1, K};
-  if (x3) p = plan_x3(false, M, N, K, split_ok, accumulate ? 1 : L.ngroup);
+  if (x3) p = plan_x3(false, M, N, K, split_ok, accumulate ? 1 : L.ngroup, !transA && transB);
   const bool once = p.ti >= 0;  // each value split once per workgroup
   if (!once) {
     p = plan_gemm(1, M, N, K, v, false, -1, bf);

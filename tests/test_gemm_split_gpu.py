@@ -208,6 +208,11 @@ def test_split_once_equals_the_split_of_every_wave(rt, form, m, n, k):
         (4100, 3080, 176),
         (16384, 384, 128),  # 128x192, whole tiles
         (300, 1028, 8192),
+        (1024, 2048, 160),  # short K: the slab-ordered kernels
+        (2048, 192, 128),
+        (256, 64, 240),  # B transposed: the waves split K where rows are no multiple of 128 bytes apart
+        (128, 448, 256),
+        (2048, 48, 1024),
     ],
 )
 def test_values_split_once_per_workgroup(rt, form, m, n, k):
