@@ -473,7 +473,9 @@ Plan plan_gemm(int batch, int M, int N, int K, int v, bool tri = false, int only
 }
 
 // ---- split products, split once per workgroup (k_gemm_x3.h) ------------------
-// The tiles with their threads, the workgroups of a CU, and the time in us
+// The tiles with their threads, the workgroups of a CU (conc_acc: of the grouped
+// products that accumulate, whose second set of sums leaves the 128-wide tiles one
+// wave per SIMD), and the time in us
 // of one 16-deep slab: of the first workgroup of a CU (lat) and of each
 // further one there (thr), and of a round's first loads and stores of C (start).
 // Measured on 16384 x 384 x 1536 and its transposes (128x192: 103-110 us for one
@@ -486,18 +488,18 @@ Plan plan_gemm(int batch, int M, int N, int K, int v, bool tri = false, int only
 // (1536 x 384 x 16384 107 us against 118).  The wide tiles split fewer values and
 // read fewer fragments per product; which of them wins is the busiest CU's
 // share of the tiles.
-struct X3Tile { int bm, bn, threads, conc; double lat, thr, start; };
-constexpr X3Tile kX3Tiles[] = {{128, 192, 256, 2, 1.0, 1.0, 7.0},
-                               {128, 128, 256, 2, 0.66, 0.66, 6.2},
-                               {256, 128, 512, 1, 1.25, 1.25, 6.5},
-                               {64, 64, 256, 4, 0.33, 0.18, 4.0}};
+struct X3Tile { int bm, bn, threads, conc, conc_acc; double lat, thr, start; };
+constexpr X3Tile kX3Tiles[] = {{128, 192, 256, 2, 1, 1.0, 1.0, 7.0},
+                               {128, 128, 256, 2, 1, 0.66, 0.66, 6.2},
+                               {256, 128, 512, 1, 1, 1.25, 1.25, 6.5},
+                               {64, 64, 256, 4, 3, 0.33, 0.18, 4.0}};
 constexpr double kX3DeepThr64 = 0.24, kX3DeepStart = 3;
 constexpr int kX3Count = sizeof(kX3Tiles) / sizeof(kX3Tiles[0]);
 constexpr int kX3K = kX3Count;  // a plan's ti: the waves split K (k_gemm_x3k.h: 32x64 tiles of eight waves)
 
 // The tile and K split with the smallest modelled time (us) of the busiest
 // CU, plus the split-K partials' round trip.
-double best_x3_tile(int M, int N, int K, bool split_ok, int groups, Plan* best) {
+double best_x3_tile(int M, int N, int K, bool split_ok, int groups, bool accumulate, Plan* best) {
   double best_t = 1e300;
   for (int ti = 0; ti < kX3Count; ++ti) {
     const X3Tile& c = kX3Tiles[ti];
@@ -512,7 +514,8 @@ double best_x3_tile(int M, int N, int K, bool split_ok, int groups, Plan* best) 
       const int kc = (int)((K + sp - 1) / sp + BK - 1) / BK * BK;
       const int ns = (K + kc - 1) / kc;
       const long per_cu = (tiles * ns + 255) / 256;
-      const long rounds = (per_cu + c.conc - 1) / c.conc;
+      const int conc = accumulate ? c.conc_acc : c.conc;
+      const long rounds = (per_cu + conc - 1) / conc;
       const double thr = K >= 1024 && c.bm == 64 ? kX3DeepThr64 : c.thr, start = K >= 1024 ? kX3DeepStart : c.start;
       double t = (kc / BK) * (rounds * c.lat + (per_cu - rounds) * thr) + rounds * start;
       if (ns > 1) t += (ns + 1.0) * M * N * groups * 4.0 / 4e6 + 3;
@@ -547,17 +550,17 @@ double x3_dma_time(int M, int N, int K, int groups) {
 // loads 16 bytes of a row of its own: 1.3 us per 8 slabs where the rows start a
 // multiple of 128 bytes apart (K = 128: 8.2 us against 6.2 on 64x64 tiles, K = 384
 // 10.8 and 10.7, K = 640 12.9 and 15.2; K = 240, whose rows do not, 6.7 and 7.5).
-Plan plan_x3(bool batched, int M, int N, int K, bool split_ok, int groups, bool nt) {
+Plan plan_x3(bool batched, int M, int N, int K, bool split_ok, int groups, bool nt, bool accumulate = false) {
   Plan best{-1, 1, K};
   read_forced_tile();
   if (g_forced_tile >= 0 || g_split_target > 0 || batched || K < 128) return best;
   if ((long)((M + 31) / 32) * ((N + 63) / 64) <= 256) {
     const int per_wave = (K / BK + 7) / 8;
     const double waves = nt && K % 32 == 0 ? per_wave * 1.3 + 7.0 : per_wave * 0.78 + (K >= 1024 ? 3.8 : 5.2);
-    if (waves < best_x3_tile(M, N, K, true, 1, &best)) return Plan{kX3K, 1, K};
+    if (waves < best_x3_tile(M, N, K, true, 1, false, &best)) return Plan{kX3K, 1, K};
   }
   const int side_by_side = split_ok ? 1 : groups;
-  const double t = best_x3_tile(M, N, K, split_ok, side_by_side, &best);
+  const double t = best_x3_tile(M, N, K, split_ok, side_by_side, accumulate, &best);
   return K < 320 && x3_dma_time(M, N, K, side_by_side) < t ? Plan{-1, 1, K} : best;
 }
 
@@ -783,7 +786,7 @@ bool gemm_grouped(int M, int N, int K, bool transA, bool transB, const GemmLayou
   const bool c_dense = L.c.r.div == 0 && L.c.c.div == 0 && L.c.c.s0 == 1 && L.c.r.s0 == N;
   const bool split_ok = !accumulate && c_dense && !(L.io & kIoC16);  // split partials are f32 and dense
   Plan p{-1, 1, K};
-  if (x3) p = plan_x3(false, M, N, K, split_ok, accumulate ? 1 : L.ngroup, !transA && transB);
+  if (x3) p = plan_x3(false, M, N, K, split_ok, accumulate ? 1 : L.ngroup, !transA && transB, accumulate);
   const bool once = p.ti >= 0;  // each value split once per workgroup
   if (!once) {
     p = plan_gemm(1, M, N, K, v, false, -1, bf);
