@@ -289,15 +289,15 @@ struct TileCfg { int tm, tn; };
 constexpr TileCfg kTiles[] = {{2, 3}, {2, 2}, {2, 1}, {1, 2}, {1, 1}};
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
-// Variant code: bit 14 = split f32 products, bits 13..9 = GemmLayouts::io
+// Variant code: bit 13 = split f32 products, bits 12..9 = GemmLayouts::io
 // (bf16-stored operands, the instances of k_gemm_io*.hip),
 // bit 8 = bf16 MFMA (autocast), bit 7 =
 // grouped accumulation, bit 6 = GELU epilogues, bit 5 = mapped operands,
 // bit 4 = LDS-DMA path, bits 3..0 = transA, transB, vecA, vecB.
 constexpr int kVarBf16 = 256;
 constexpr int kVarIoShift = 9;
-constexpr int kVarX3 = 1 << 14;  // f32 product as split bf16 pieces (LDS-DMA kernels)
-constexpr int kVarCount = 1 << 15;
+constexpr int kVarX3 = 1 << 13;  // f32 product as split bf16 pieces (LDS-DMA kernels)
+constexpr int kVarCount = 1 << 14;
 inline int variant(bool ta, bool tb, bool va, bool vb, bool dma) {
   return (dma << 4) | (ta << 3) | (tb << 2) | (va << 1) | (int)vb;
 }
@@ -352,7 +352,7 @@ const void* kernel_for_prec(int ti, int v) {
 }
 
 const void* kernel_for(int ti, int v) {
-  if ((v >> kVarIoShift) & 31) return gemm_io_kernel(ti, v);
+  if ((v >> kVarIoShift) & 15) return gemm_io_kernel(ti, v);
   if (v & kVarX3) return kernel_for_prec<2>(ti, v);
   return (v & kVarBf16) ? kernel_for_prec<1>(ti, v) : kernel_for_prec<0>(ti, v);
 }
@@ -652,8 +652,8 @@ double launch_dma(const float* A, const float* B, float* C, int batch, int M, in
   Plan p{-1, 1, K};
   // a product of batches has a batch stride, whatever the number of batches
   const auto strided = [](const GemmMap& b) { return b.s0 != 0 || b.s1 != 0; };
-  const bool batched = batch > 1 || strided(L.a.b) || strided(L.b.b);
-  if (x3 && !(mapped && L.tri_a)) p = plan_x3(batched, M, N, K, split_ok, 1, !transA && transB);
+  const bool batched = batch > 1 || strided(L.a.b) || strided(L.b.b), both = transA && transB;
+  if (x3 && !both && !(mapped && L.tri_a)) p = plan_x3(batched, M, N, K, split_ok, 1, !transA && transB);
   const bool once = p.ti >= 0;  // each value split once per workgroup
   if (!once) {
     // Under autocast the GELU GEMM (h = x W1, K = 384, a 3072-workgroup grid
@@ -662,7 +662,8 @@ double launch_dma(const float* A, const float* B, float* C, int batch, int M, in
     if (!split_ok && p.nsplit > 1) p = Plan{p.ti, 1, K};
   }
   int wide_bf = -1;
-  if (bf && !L.io && !mapped && !epi && batch == 1 && g_forced_tile < 0) wide_bf = plan_bf(M, N, p, transA && K >= 4096);
+  if (bf && !L.io && !both && !mapped && !epi && batch == 1 && g_forced_tile < 0)
+    wide_bf = plan_bf(M, N, p, transA && K >= 4096);
   const TileShape ts = wide_bf >= 0 ? TileShape{256, wide_bf ? 128 : 256, 512} : tile_shape(once, p.ti);
   trace_plan(batch, M, N, K, transA, transB, wide_bf >= 0 ? "bf" : once ? "x3" : "dma", p, ts, mapped ? " mapped" : "");
   const int bm = ts.bm, bn = ts.bn;
@@ -786,7 +787,7 @@ bool gemm_grouped(int M, int N, int K, bool transA, bool transB, const GemmLayou
   const bool c_dense = L.c.r.div == 0 && L.c.c.div == 0 && L.c.c.s0 == 1 && L.c.r.s0 == N;
   const bool split_ok = !accumulate && c_dense && !(L.io & kIoC16);  // split partials are f32 and dense
   Plan p{-1, 1, K};
-  if (x3) p = plan_x3(false, M, N, K, split_ok, accumulate ? 1 : L.ngroup, !transA && transB, accumulate);
+  if (x3 && !(transA && transB)) p = plan_x3(false, M, N, K, split_ok, accumulate ? 1 : L.ngroup, !transA && transB, accumulate);
   const bool once = p.ti >= 0;  // each value split once per workgroup
   if (!once) {
     p = plan_gemm(1, M, N, K, v, false, -1, bf);

@@ -145,7 +145,7 @@ __device__ __forceinline__ void write16(float* P, const v16f& v, Live&& live, Of
 // whose div is a multiple of 32, 16-byte aligned k-contiguous rows, and byte
 // offsets below 2^31.  WM x WN waves of TM x TN accumulators.
 template <int WM, int WN, int TM, int TN, bool TA, bool TB, bool MAP, int EPI, int G = 1>
-__global__ __launch_bounds__(64 * WM * WN, WM * WN == 4 && (EPI == 3 || TM * TN > 8) ? 1 : 2) void k_gemm_x3(const float* __restrict__ A,
+__global__ __launch_bounds__(64 * WM * WN, WM * WN == 4 && EPI == 3 ? 1 : 2) void k_gemm_x3(const float* __restrict__ A,
                                                                          const float* __restrict__ B,
                                                                          float* __restrict__ C, int M, int N, int K,
                                                                          GemmLayouts L, int k_chunk, int tiles_n,

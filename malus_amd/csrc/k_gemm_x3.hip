@@ -8,8 +8,9 @@ namespace malus {
 namespace k {
 namespace {
 
-// Variant bits as in k_gemm.hip: 8 transA, 4 transB, 32 mapped operands,
-// 64 GELU epilogues, 128 grouped accumulation.
+// Variant bits as in k_gemm.hip: 8 transA, 4 transB (the planner sends no
+// product with both here), 32 mapped operands, 64 GELU epilogues, 128 grouped
+// accumulation.
 template <int WM, int WN, int TM, int TN, int G>
 const void* x3_instance(int v) {
 #define MALUS_X3(TA, TB, MAP, EPI) reinterpret_cast<const void*>(&k_gemm_x3<WM, WN, TM, TN, TA, TB, MAP, EPI, G>)
@@ -17,10 +18,10 @@ const void* x3_instance(int v) {
   if (v & 128) return !ta && tb ? MALUS_X3(false, true, true, 3) : nullptr;
   if (v & 64) return ta ? nullptr : tb ? MALUS_X3(false, true, false, 2) : MALUS_X3(false, false, false, 1);
   if (mapped) {
-    if (ta) return tb ? MALUS_X3(true, true, true, 0) : MALUS_X3(true, false, true, 0);
+    if (ta) return MALUS_X3(true, false, true, 0);
     return tb ? MALUS_X3(false, true, true, 0) : MALUS_X3(false, false, true, 0);
   }
-  if (ta) return tb ? MALUS_X3(true, true, false, 0) : MALUS_X3(true, false, false, 0);
+  if (ta) return MALUS_X3(true, false, false, 0);
   return tb ? MALUS_X3(false, true, false, 0) : MALUS_X3(false, false, false, 0);
 #undef MALUS_X3
 }
@@ -42,10 +43,10 @@ const void* gemm_x3k_kernel(int v) {
   if (v & 128) return !ta && tb ? MALUS_X3K(false, true, true, 3) : nullptr;
   if (v & 64) return ta ? nullptr : tb ? MALUS_X3K(false, true, false, 2) : MALUS_X3K(false, false, false, 1);
   if (mapped) {
-    if (ta) return tb ? MALUS_X3K(true, true, true, 0) : MALUS_X3K(true, false, true, 0);
+    if (ta) return MALUS_X3K(true, false, true, 0);
     return tb ? MALUS_X3K(false, true, true, 0) : MALUS_X3K(false, false, true, 0);
   }
-  if (ta) return tb ? MALUS_X3K(true, true, false, 0) : MALUS_X3K(true, false, false, 0);
+  if (ta) return MALUS_X3K(true, false, false, 0);
   return tb ? MALUS_X3K(false, true, false, 0) : MALUS_X3K(false, false, false, 0);
 #undef MALUS_X3K
 }
@@ -53,9 +54,7 @@ const void* gemm_x3k_kernel(int v) {
 template <int WM, int WN, int TM, int TN, int G>
 const void* bf_instance(int v) {
   const bool ta = v & 8, tb = v & 4;
-  if (ta)
-    return tb ? reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, true, true, G>)
-              : reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, true, false, G>);
+  if (ta) return reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, true, false, G>);
   return tb ? reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, false, true, G>)
             : reinterpret_cast<const void*>(&k_gemm_bf<WM, WN, TM, TN, false, false, G>);
 }
