@@ -114,24 +114,7 @@ struct Tile {
   }
   // 4 values (columns 4 c4 ..) of row r
   __device__ __forceinline__ static void store(char* S, int r, int c4, v4f f) {
-    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-    char* at = S + r * ROW + (((c4 >> 1) ^ swz(r)) << 4) + ((c4 & 1) << 3);
-    unsigned h[2], m[2], l[2];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const float a = f[2 * q], b = f[2 * q + 1];
-      h[q] = pack_bf16(a, b);
-      if constexpr (NP == 3) {
-        const float ra = a - bf16_low(h[q]), rb = b - bf16_high(h[q]);
-        m[q] = pack_bf16(ra, rb);
-        l[q] = pack_bf16(ra - bf16_low(m[q]), rb - bf16_high(m[q]));
-      }
-    }
-    *reinterpret_cast<u32x2*>(at) = u32x2{h[0], h[1]};
-    if constexpr (NP == 3) {
-      *reinterpret_cast<u32x2*>(at + PLANE) = u32x2{m[0], m[1]};
-      *reinterpret_cast<u32x2*>(at + 2 * PLANE) = u32x2{l[0], l[1]};
-    }
+    store_planes<NP>(S + r * ROW + (((c4 >> 1) ^ swz(r)) << 4) + ((c4 & 1) << 3), PLANE, {f[0], f[1], f[2], f[3]});
   }
   // columns 16 kb + 8 lk .. of row r (the lane's own lk)
   __device__ __forceinline__ static Frag<NP> row(const char* S, int r, int kb, int lk) {

@@ -78,23 +78,7 @@ struct X3Stage {
   }
   // splits (rounds) unit u's values into the planes at S
   __device__ __forceinline__ void store(char* S, int u, v4f f) const {
-    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-    unsigned h[2], m[2], l[2];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const float a = f[2 * q], b = f[2 * q + 1];
-      h[q] = pack_bf16(a, b);
-      if constexpr (NP == 3) {
-        const float ra = a - bf16_low(h[q]), rb = b - bf16_high(h[q]);
-        m[q] = pack_bf16(ra, rb);
-        l[q] = pack_bf16(ra - bf16_low(m[q]), rb - bf16_high(m[q]));
-      }
-    }
-    *reinterpret_cast<u32x2*>(S + loff[u]) = u32x2{h[0], h[1]};
-    if constexpr (NP == 3) {
-      *reinterpret_cast<u32x2*>(S + PLANE + loff[u]) = u32x2{m[0], m[1]};
-      *reinterpret_cast<u32x2*>(S + 2 * PLANE + loff[u]) = u32x2{l[0], l[1]};
-    }
+    store_planes<NP>(S + loff[u], PLANE, {f[0], f[1], f[2], f[3]});
   }
 #endif
 };

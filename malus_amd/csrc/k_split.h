@@ -45,6 +45,40 @@ __device__ __forceinline__ unsigned pack_bf16(float a, float b) {
 __device__ __forceinline__ float bf16_low(unsigned p) { return __builtin_bit_cast(float, p << 16); }
 __device__ __forceinline__ float bf16_high(unsigned p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
 
+// The pieces of two values, packed: every split in the library is made of
+// this one.
+__device__ __forceinline__ void split_pair(float a, float b, unsigned& h, unsigned& m, unsigned& l) {
+  h = pack_bf16(a, b);
+  const float ra = a - bf16_low(h), rb = b - bf16_high(h);
+  m = pack_bf16(ra, rb);
+  l = pack_bf16(ra - bf16_low(m), rb - bf16_high(m));
+}
+
+// Four values in NP planes at S (8 bytes each, `plane` bytes apart): the three
+// pieces, or for NP = 1 the values rounded to bf16.
+template <int NP>
+__device__ __forceinline__ void store_planes(char* S, int plane, const float (&f)[4]) {
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  u32x2 h, m, l;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    if constexpr (NP == 3) {
+      unsigned a, b, c;
+      split_pair(f[2 * q], f[2 * q + 1], a, b, c);
+      h[q] = a;
+      m[q] = b;
+      l[q] = c;
+    } else {
+      h[q] = pack_bf16(f[2 * q], f[2 * q + 1]);
+    }
+  }
+  *reinterpret_cast<u32x2*>(S) = h;
+  if constexpr (NP == 3) {
+    *reinterpret_cast<u32x2*>(S + plane) = m;
+    *reinterpret_cast<u32x2*>(S + 2 * plane) = l;
+  }
+}
+
 // The three pieces of a lane's 8 fragment values, packed as the MFMA reads
 // them (value e in half-word e).
 struct Split3 {
@@ -54,12 +88,7 @@ struct Split3 {
 __device__ __forceinline__ Split3 split3(const float (&f)[8]) {
   unsigned hp[4], mp[4], lp[4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    hp[q] = pack_bf16(f[2 * q], f[2 * q + 1]);
-    const float ra = f[2 * q] - bf16_low(hp[q]), rb = f[2 * q + 1] - bf16_high(hp[q]);
-    mp[q] = pack_bf16(ra, rb);
-    lp[q] = pack_bf16(ra - bf16_low(mp[q]), rb - bf16_high(mp[q]));
-  }
+  for (int q = 0; q < 4; ++q) split_pair(f[2 * q], f[2 * q + 1], hp[q], mp[q], lp[q]);
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
   return Split3{__builtin_bit_cast(bf16x8, (u32x4){hp[0], hp[1], hp[2], hp[3]}),
                 __builtin_bit_cast(bf16x8, (u32x4){mp[0], mp[1], mp[2], mp[3]}),
