@@ -1,5 +1,6 @@
 """Headline benchmark: warm-median ms/step of the Karpathy char-nanoGPT f32
-training step on one MI355X.
+training step (batch 64, block 256, embedding 384, 6 heads, 6 layers) on one
+MI355X.
 
 A step = token upload (the `freeze` of buffer.rs:39-50) -> zero_grad ->
 forward -> cross_entropy -> backward -> "AdamW" (examples/nanogpt_modular.ml:
@@ -8,8 +9,8 @@ step (docs/adr/0038-benchmark-methodology.md).  Token batches are synthetic
 (int32 i.i.d. uniform in [0, 65) from a fixed seed), built on the host before
 timing and uploaded inside each timed step.  Prints ONE JSON line.
 
---config c4 runs the toy char-nanoGPT the same
-way; --config c1 runs the XOR MLP's 10,000 steps.
+--config c4 runs the toy char-nanoGPT (batch 32, block 64, embedding 128, 4
+heads, 4 layers) the same way; --config c1 runs the XOR MLP's 10,000 steps.
 """
 from __future__ import annotations
 
@@ -104,8 +105,7 @@ def copy_calibration(rt, sizes):
 def kernel_suite(rt, M, reps: int):
     """C2 (elementwise, 2^26 f32) and C3 (row ops on [65536, 1024]) kernels
     through the C ABI, each timed over `reps` launches between device
-    flushes; bandwidth = algorithmic bytes / time (
-    configs[2]).  Returns a list of rows; prints a table to stderr."""
+    flushes; bandwidth = algorithmic bytes / time.  Returns a list of rows; prints a table to stderr."""
     import numpy as np
 
     L = rt.L

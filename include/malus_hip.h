@@ -375,8 +375,7 @@ int64_t malus_gpt_logits(void* g, int64_t toks);
 void malus_gpt_zero_grad(void* g);
 void malus_gpt_optimizer_step(void* g, int64_t t);    /* nanogpt_modular.ml:186-188 */
 int64_t malus_gpt_step(void* g, int64_t toks, int64_t targets, int64_t t); /* nanogpt_modular.ml:167-189 */
-/* No reference counterpart: the whole training step as a HIP graph (the
- * "optionally hipGraph-captured train steps" of the north star).  create runs
+/* No reference counterpart: the whole training step as a HIP graph.  create runs
  * step t eagerly (its loss in *loss_out) and captures the step; each
  * graph_step replays it for step t on new token/target ids (copied from
  * pinned host memory by the graph's own nodes) and returns the loss tensor

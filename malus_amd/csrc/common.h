@@ -149,9 +149,9 @@ struct BcastDesc {          // NumPy right-aligned broadcast of (p op q) into ou
   uint32_t q_stride[kMaxRank];
 };
 
-// out[i] = p[i] op q[i]
 // out = old + p * q (the product rounded to f32 before the add).
 void mul_add(const float* p, const float* q, const float* old, float* out, size_t n, hipStream_t s);
+// out[i] = p[i] op q[i]
 void binary_same(int op, const float* p, const float* q, float* out, size_t n, hipStream_t s);
 // out = p op q with q broadcast along rows: q_flat = i % qn (trailing-block broadcast)
 void binary_rowbcast(int op, const float* p, const float* q, float* out, size_t n, size_t qn, hipStream_t s);

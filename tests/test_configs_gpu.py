@@ -1,14 +1,14 @@
 """The C2 and C3 workloads as programs through the tape (their composed
 chains, not each op on its own), and C5 over several steps.
 
-C2 (BASELINE configs[1]): z = a*b + 0.5*c - relu(a) and a [R,C] + [1,C] row
+C2: z = a*b + 0.5*c - relu(a) and a [R,C] + [1,C] row
 broadcast, forward and backward.  The tensor-scalar product `0.5*c` records
 no tape node (codegen-cpu/src/lib.rs:1556-1580), so c receives no gradient;
 the other gradients are sums of +-1, b and a and come out bit-exact.
 
 Both run at the configuration's own [8192, 8192] and at 1/64 of it.
 
-C3 (configs[2]), at [65536, 1024]: layernorm with gamma = 1 and beta = 0
+C3, at [65536, 1024]: layernorm with gamma = 1 and beta = 0
 perturbed by N(0, 0.02) (nanogpt_modular.ml:38-45 applies the weight as a
 broadcast mul), through the tape with a random upstream gradient: normwise
 1e-5 against the oracle's composition of the same VJPs (also at 4,096 rows);
@@ -16,7 +16,7 @@ softmax, GELU and cross-entropy (logits ~ N(0, 2), int32 targets in
 [0, 1024)) forward and backward, and the axis-0 and axis-1 sums, against the
 oracle at the bars of tests/helpers.py.
 
-C5 (configs[4]): three training steps (loss within 1e-5 relative each step;
+C5: three training steps (loss within 1e-5 relative each step;
 after the third, at most 0.1% of the parameters more than 1e-5 apart)."""
 import ctypes as C
 import os

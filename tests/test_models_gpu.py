@@ -1,6 +1,6 @@
 """End-to-end parity of the workload drivers against the CPU oracle:
 examples/xor.ml (C1), the toy char-nanoGPT (C4) and the Karpathy
-char-nanoGPT (C5).  Loss trajectories: within 1e-3 relative (north star);
+char-nanoGPT (C5).  Loss trajectories: within 1e-3 relative;
 single-step gradients: normwise 3e-5 (per-op 1e-5 errors compound through
 ~40 dependent ops per block; measured worst 2.5e-6 at C4, 7.0e-6 at C5)."""
 import ctypes as C
@@ -332,7 +332,7 @@ def _c5_corpus_losses(rt, steps, autocast):
 
 
 def test_gpt_c5_200_step_trajectory_vs_oracle_fixture(rt):
-    """The north star's trajectory bar on the configuration's own data: 200
+    """The 1e-3 trajectory bar on the configuration's own data: 200
     replays of the captured C5 step, each drawing its i.i.d. ids on the
     device (the bench's path), every loss within 1e-3 relative of the CPU
     oracle's (tests/golden/c5_trajectory_iid.json)."""
