@@ -52,8 +52,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_bf(const float* __rest
     if ((nt & 7) == 0) tile = (tile & 7) * (nt >> 3) + (tile >> 3);
     split = 0;
   } else {
-    const int total = nt * ns, lin = blockIdx.x + nt * blockIdx.y;
-    const int w = (total & 7) == 0 ? (lin & 7) * (total >> 3) + (lin >> 3) : lin;
+    const int w = xcd_range(blockIdx.x + nt * blockIdx.y, nt * ns);
     split = __builtin_amdgcn_readfirstlane(w / nt);
     tile = w - split * nt;
   }

@@ -31,6 +31,16 @@ typedef float v4f_raw __attribute__((ext_vector_type(4)));  // 4 words of packed
 
 constexpr int BK = 16;
 
+// Workgroup `lin` of a launch of `total` runs on XCD lin % 8 (dispatch deals
+// them round robin): the lin-th entry of a list of which every XCD takes one
+// contiguous range, the ranges differing by at most one entry.  A one-to-one map
+// for any total; without it, 252 workgroups of the weight gradients (36 tiles
+// by 7 splits) left every XCD all of K and fetched 2-4 times their operands.
+__host__ __device__ constexpr int xcd_range(int lin, int total) {
+  const int x = lin & 7, rest = total & 7;
+  return x * (total >> 3) + (x < rest ? x : rest) + (lin >> 3);
+}
+
 // The MFMA work of one 16-deep K step from each lane's 8 fragment values
 // (k = 8h + s for lane half h, the same k slots in A and B): eight FP32
 // 32x32x2 steps, or under autocast (BF) one 32x32x16 bf16 MFMA over the same
