@@ -57,7 +57,8 @@ __device__ __forceinline__ v16f mul(const Frag<NP>& a, const Frag<NP>& b, v16f c
 // instructions where expf, which also clamps its range, takes 13.  As accurate
 // as expf, under autocast too: the f32 row sums and the log-sum-exp are made of
 // these values, and without the correction their error grows with |x| (rms
-// 4e-7 of the value at x = -20 .. -10, 2e-6 at -80 .. -40, against 2.5e-8).
+// 4e-7 of the value at x = -20 .. -10, 2e-6 at -80 .. -40, against 2.5e-8; 48
+// heads, T = 2048, autocast, forward + backward 219 us without, 247 with).
 // The correction is NaN at an infinite x; fmaxf makes a factor of the zero power
 // of it where x is never above 0 (LE0: behind the row's maximum).  Elsewhere a
 // negative correction would also make NaN of an infinite power, so where 2^p is

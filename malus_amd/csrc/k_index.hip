@@ -414,7 +414,8 @@ void embedding_bwd(const float* dout, const int32_t* idx, float* dw, size_t t, s
 // Up to here (256 KiB, at most 256 workgroups) k_transpose_small's strided
 // reads stay in cache and it is the faster one at every shape tried: [4, 8] 3.1 ->
 // 1.6 us, [64, 64] 5.1 -> 2.1, [32, 512] 4.5 -> 2.2, [256, 256] 5.5 -> 2.4,
-// [4, 65, 128] 5.6 -> 2.3 (kernel time).
+// [4, 65, 128] 5.6 -> 2.3 (kernel time; a call by itself is bound by its launch, [4,
+// 8] 3.85 -> 3.75).
 constexpr size_t kSmallTranspose = 65536;
 
 void permute(const float* x, float* out, int ndim, const size_t* in_shape, const size_t* perm, hipStream_t s) {
