@@ -52,25 +52,22 @@ __device__ __forceinline__ v16f mul(const Frag<NP>& a, const Frag<NP>& b, v16f c
   else return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[0], b.p[0], c, 0, 0, 0);
 }
 
-// exp(x): 2^p for p = x log2(e) rounded, corrected by the first order of
-// what the rounding left (x - p ln 2, exact but for its last bits): 6 or 7
-// instructions where expf, which also clamps its range, takes 13.  As accurate
-// as expf, under autocast too: the f32 row sums and the log-sum-exp are made of
-// these values, and without the correction their error grows with |x| (rms
-// 4e-7 of the value at x = -20 .. -10, 2e-6 at -80 .. -40, against 2.5e-8; 48
-// heads, T = 2048, autocast, forward + backward 219 us without, 247 with).
-// The correction is NaN at an infinite x; fmaxf makes a factor of the zero power
-// of it where x is never above 0 (LE0: behind the row's maximum).  Elsewhere a
-// negative correction would also make NaN of an infinite power, so where 2^p is
-// infinite or (below 2^-126) zero the factor is 1.
-template <bool LE0>
+// exp(x) = 2^n 2^f, n the integer nearest x log2(e) and f the rest from two
+// fused multiply-adds (log2(e) = 1.44269502 + 1.92596299e-8): 8 instructions
+// where expf takes 13, and its accuracy (rms 2.67e-8 of the value and at most 8.6e-8
+// over x = -80 .. 0, expf 2.63e-8 and 8.4e-8; both are v_exp_f32's own error).
+// Under autocast too: the f32 row sums and the log-sum-exp are made of these
+// values.  Shorter forms measured worse: 2^(x log2(e)) in two instructions 4.2e-7
+// at x = -20 .. -10 and 1.7e-6 at -80 .. -40, the same corrected behind v_exp_f32 in
+// six 3.6e-8 and 1.4e-7 at most.  48 heads, T = 2048, autocast, forward + backward:
+// 219 us with two instructions, 250 with six, 263 here, 296 with expf; 384 heads,
+// T = 256, f32: 150.2 with six, 150.4 here, 153.8 with expf.  The clamp keeps n an
+// integer that ldexp takes; f is then infinite where x is, and NaN where x is.
 __device__ __forceinline__ float exp_of(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  const float p = x * 1.44269504f;
-  const float e = __builtin_amdgcn_exp2f(p);
-  // ln 2 = 0.693147182 - 1.90465421e-9
-  const float c = __builtin_fmaf(p, 1.90465421e-9f, __builtin_fmaf(p, -0.693147182f, x));
-  return __builtin_fmaf(e, LE0 ? fmaxf(c, -1.0f) : __builtin_fabsf(p) < 128.0f ? c : 1.0f, e);
+  const float n = __builtin_rintf(__builtin_amdgcn_fmed3f(x * 1.44269504f, -160.0f, 160.0f));
+  const float f = __builtin_fmaf(x, 1.92596299e-8f, __builtin_fmaf(x, 1.44269504f, -n));
+  return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
 #else
   return x;
 #endif
@@ -248,7 +245,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_fwd(const float* __r
       float ls = 0.0f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float p = exp_of<true>(st[r] - mn);
+        const float p = exp_of(st[r] - mn);
         st[r] = p;
         ls += p;
       }
@@ -369,7 +366,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dq(const float* __re
         dp = mul<NP>(Tl::row(Vs[cur], perm_row(x), kb, lk), og[kb], dp);
       }
 #pragma unroll
-      for (int r = 0; r < 16; ++r) st[r] = exp_of<false>(st[r] * sc - L);
+      for (int r = 0; r < 16; ++r) st[r] = exp_of(st[r] * sc - L);
       if (CAUSAL && j == qt) {
 #pragma unroll
         for (int r = 0; r < 16; ++r)
@@ -499,7 +496,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_flash_planes_dkv(
       }
       // lane = key j0 + x, register r = query i0 + perm_index(r, lk)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = exp_of<false>(s[r] * sc - Ls[cur][0][perm_index(r, lk)]);
+      for (int r = 0; r < 16; ++r) s[r] = exp_of(s[r] * sc - Ls[cur][0][perm_index(r, lk)]);
       if (CAUSAL && it == kt) {
 #pragma unroll
         for (int r = 0; r < 16; ++r)
