@@ -10,11 +10,10 @@
 // tile: its f32 values are loaded once per workgroup, split once and kept in
 // LDS as bf16 planes.  With four waves (AHEAD) the planes are double buffered,
 // the next tile's loads are in flight during the current tile's products and a
-// tile takes one barrier.  Workgroups of one or two waves, which have a tile or
-// two to stream, keep one buffer and load between the products: the registers
-// and the LDS of the second stage cost them more waves per CU than it hides
-// (dkv at head size 64 spilled 31 registers; see dispatch for the times).  Both
-// orientations are read from the same planes: rows with 128-bit reads,
+// tile takes one barrier.  Workgroups of one or two waves keep one buffer and
+// load between the products: the registers and the LDS of the second stage cost
+// them more waves per CU than it hides (dkv at head size 64 spilled 31
+// registers; the times stand at group_waves).  Both orientations are read from the same planes: rows with 128-bit reads,
 // columns with gfx950's transposing read (ds_read_b64_tr_b16).
 // The products run in the order of the per-wave form; only exp differs (exp_of).
 #include "k_flash.h"

@@ -242,3 +242,30 @@ def test_c4_bf16_activations_equal_f32_storage(rt, attention):
     assert runs[True][0] == runs[False][0]
     for i, (a, b) in enumerate(zip(runs[True][1], runs[False][1])):
         assert np.array_equal(bits(a), bits(b)), f"state tensor {i} differs"
+
+
+@pytest.mark.parametrize("t,c,h", [(32, 128, 4), (32, 128, 2), (64, 128, 2), (96, 128, 4), (160, 256, 4)])
+def test_short_sequences_bf16_storage_equal_f32_storage(rt, t, c, h):
+    """Flash attention on bf16 q, k, v with one, two and four 32-row tiles a
+    workgroup (whole and ragged groups), head sizes 32 and 64: two steps equal
+    those on f32 storage, bit for bit."""
+    cfg = dict(V=65, T=t, C=c, H=h, L=1, B=4)
+    n = cfg["B"] * t
+    x, y = O.rand_tokens(9 << 32, n, 65), O.rand_tokens((9 << 32) + n, n, 65)
+    runs = []
+    with M.autocast():
+        for on in (True, False):
+            g = _make(rt, cfg, on)
+            assert rt.L.malus_gpt_set_attention(g, 1) == 0
+            losses = []
+            for k in (1, 2):
+                hx, hy = rt.tensor(x), rt.tensor(y)
+                hl = rt.L.malus_gpt_step(g, hx, hy, k)
+                losses.append(rt.numpy(hl)[0])
+                rt.free(hl, hx, hy)
+            runs.append((losses, _state(rt, g)))
+            rt.L.malus_gpt_free(g)
+            rt.L.tape_reset()
+    assert runs[0][0] == runs[1][0]
+    for i, (a, b) in enumerate(zip(runs[0][1], runs[1][1])):
+        assert np.array_equal(bits(a), bits(b)), f"state tensor {i} differs"
